@@ -966,7 +966,9 @@ int Flow<D>::probe(int which, int reps, double *avg_ms, long *bytes) {
             // the symmetric velocity systems of uniform meshes)
             (void)hipEventDestroy(a);
             (void)hipEventDestroy(b);
-            if (!hbatched_ || !hsysB_.k32.amg_on()) return -1;
+            if (!hbatched_) return -1;
+            hsysB_.ensure_amg(st_);
+            if (!hsysB_.k32.amg_on()) return -1;
             const float ms = hsysB_.k32.amg.probe_pp(reps, &by, st_);
             if (ms < 0) return -1;
             *avg_ms = ms;
@@ -979,6 +981,7 @@ int Flow<D>::probe(int which, int reps, double *avg_ms, long *bytes) {
             // the fine-level residual launch of its FP64 V-cycle (15)
             (void)hipEventDestroy(a);
             (void)hipEventDestroy(b);
+            psys_.ensure_amg(st_);
             const float ms = which == 14 ? (psys_.k32.amg_on() ? psys_.k32.amg.probe_pp(reps, &by, st_) : -1.0f)
                                          : (psys_.k64.amg_on() ? psys_.k64.amg.probe_resid(reps, &by, st_) : -1.0f);
             if (ms < 0) return -1;

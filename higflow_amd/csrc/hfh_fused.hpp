@@ -31,6 +31,7 @@ class FusedKrylov {
     // BiCGStab right-preconditioned by a smoothed-aggregation V-cycle
     // (requested before set(); used when the hierarchy builds)
     bool want_amg = false;
+    bool defer_amg = false;  // set() leaves the hierarchy to build_amg()
     double amg_max_cx = 0;  // > 0: no hierarchy above this operator complexity
     AmgPrecond<T> amg;
     // symmetric systems with a hierarchy: AMG-PCG (HFH_AMG_PCG=0: AMG-BiCGStab)
@@ -108,6 +109,11 @@ class FusedKrylov {
         k_fill<T><<<nblocks((long)KS_N * nseg), BLOCK, 0, st>>>(KS_N * nseg, ks.p, T(0));
         k_fill<int><<<nblocks((long)KI_N * nseg), BLOCK, 0, st>>>(KI_N * nseg, ki.p, 0);
         amg.ready = false;
+        if (!defer_amg) build_amg(hrp, hci, hv, st);
+    }
+    // the V-cycle of the matrix set() took (with defer_amg: on first use)
+    void build_amg(const std::vector<int> &hrp, const std::vector<int> &hci, const std::vector<double> &hv,
+                   hipStream_t st) {
         {
             const char *e = std::getenv("HFH_AMG_PCG");
             amg_pcg = !(e && std::strcmp(e, "0") == 0);

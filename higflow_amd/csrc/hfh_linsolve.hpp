@@ -25,6 +25,7 @@
 
 #include "hfh_kernels.hpp"
 #include "hfh_fused.hpp"
+#include "hfh_fdm.hpp"
 
 #define HFH_CHECK(x)                                                                        \
     do {                                                                                    \
@@ -347,54 +348,60 @@ __global__ void __launch_bounds__(BLOCK) k_residual(int n, const int *__restrict
 }
 
 // the same with 4 lanes per row: workgroups of 4 BLOCK threads, one per
-// BLOCK rows, so the partials have k_residual's layout (one per BLOCK rows)
+// BLOCK rows, so the partials have k_residual's layout (one per BLOCK rows);
+// prs: the sums of r
 template <typename T>
 __global__ void __launch_bounds__(4 * BLOCK) k_residual_l4(int n, const int *__restrict__ rp,
                                                            const int *__restrict__ ci, const T *__restrict__ v,
                                                            const T *__restrict__ x, const T *__restrict__ b,
                                                            T *__restrict__ r, T *__restrict__ prr,
-                                                           T *__restrict__ pbb) {
+                                                           T *__restrict__ pbb, T *__restrict__ prs) {
     const int i = blockIdx.x * BLOCK + (int)threadIdx.x / 4, lane = threadIdx.x & 3;
     T s = 0;
     if (i < n)
         for (int k = rp[i] + lane; k < rp[i + 1]; k += 4) s += v[k] * x[ci[k]];
     s += __shfl_xor(s, 1, 64);
     s += __shfl_xor(s, 2, 64);
-    T rr = 0, bb = 0;
+    T rr = 0, bb = 0, rs = 0;
     if (i < n && lane == 0) {
         const T bi = b[i], ri = bi - s;
         r[i] = ri;
         rr = ri * ri;
         bb = bi * bi;
+        rs = ri;
     }
     rr = wave_sum(rr);
     bb = wave_sum(bb);
-    __shared__ T srr[4 * BLOCK / 64], sbb[4 * BLOCK / 64];
+    rs = wave_sum(rs);
+    __shared__ T srr[4 * BLOCK / 64], sbb[4 * BLOCK / 64], srs[4 * BLOCK / 64];
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
         srr[w] = rr;
         sbb[w] = bb;
+        srs[w] = rs;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        T a = 0, c = 0;
+        T a = 0, c = 0, e = 0;
         for (int q = 0; q < 4 * BLOCK / 64; q++) {
             a += srr[q];
             c += sbb[q];
+            e += srs[q];
         }
         prr[blockIdx.x] = a;
         pbb[blockIdx.x] = c;
+        prs[blockIdx.x] = e;
     }
 }
 
 // r = b - A x with the matrix in the diagonal form of the Krylov kernels
 // (KRows::dblk; rows without a template read CSR), one row per thread in
-// 1024-row workgroups; partials r.r and b.b per 256-row block as
+// 1024-row workgroups; partials r.r, b.b and sum(r) per 256-row block as
 // k_residual_l4 writes them (one per BLOCK rows, nb of them).
 template <typename T>
 __global__ void __launch_bounds__(KNT) k_residual_d(int n, KRows<T> A, const T *__restrict__ x,
                                                     const T *__restrict__ b, T *__restrict__ r, T *__restrict__ prr,
-                                                    T *__restrict__ pbb, int nb) {
+                                                    T *__restrict__ pbb, T *__restrict__ prs, int nb) {
     const int i = blockIdx.x * KNT + (int)threadIdx.x;
     const bool in = i < n;
     const int *db = A.dblk + (size_t)blockIdx.x * (KD_MAX + 1);
@@ -419,33 +426,38 @@ __global__ void __launch_bounds__(KNT) k_residual_d(int n, KRows<T> A, const T *
     } else if (in) {
         for (int k = A.rp[i]; k < A.rp[i + 1]; k++) s += A.val[k] * x[A.ci[k]];
     }
-    T rr = 0, bb = 0;
+    T rr = 0, bb = 0, rs = 0;
     if (in) {
         const T bi = b[i], ri = bi - s;
         r[i] = ri;
         rr = ri * ri;
         bb = bi * bi;
+        rs = ri;
     }
     rr = wave_sum(rr);
     bb = wave_sum(bb);
-    __shared__ T srr[KNT / 64], sbb[KNT / 64];
+    rs = wave_sum(rs);
+    __shared__ T srr[KNT / 64], sbb[KNT / 64], srs[KNT / 64];
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
         srr[w] = rr;
         sbb[w] = bb;
+        srs[w] = rs;
     }
     __syncthreads();
     constexpr int WPB = BLOCK / 64;  // waves per 256-row block
     if (threadIdx.x < KNT / BLOCK) {
         const int q = threadIdx.x, pb = blockIdx.x * (KNT / BLOCK) + q;
-        T a = 0, c = 0;
+        T a = 0, c = 0, e = 0;
         for (int k = 0; k < WPB; k++) {
             a += srr[q * WPB + k];
             c += sbb[q * WPB + k];
+            e += srs[q * WPB + k];
         }
         if (pb < nb) {
             prr[pb] = a;
             pbb[pb] = c;
+            prs[pb] = e;
         }
     }
 }
@@ -497,6 +509,7 @@ class DeviceSystem {
     // fused iterations (FP64 solve and FP32 inner solve of the mixed form)
     FusedKrylov<double> k64;
     FusedKrylov<float> k32;
+    FdmSolver fdm;  // direct solves of Kronecker-sum matrices
     bool fused = true;
     int max_restarts = 1;      // fused64: restarts on the true residual
     double t_mixed_ = -1, t_fp64_ = -1;  // mixed form: seconds per solve of each form
@@ -573,7 +586,8 @@ class DeviceSystem {
         off_ks_ = ((nseg * KI_N * (int)sizeof(int) + 63) / 64) * 64;
         off_sc_ = off_ks_ + ((nseg * KS_N * (int)sizeof(double) + 63) / 64) * 64;
         off_rr_ = off_sc_ + 256;
-        const size_t pin = (size_t)off_rr_ + 2 * (size_t)nb * sizeof(double);
+        off_fd_ = off_rr_ + 2 * nb * (int)sizeof(double);
+        const size_t pin = (size_t)off_fd_ + 2 * (size_t)nseg * sizeof(double);
         clear_graphs();
         {
             // off by default: on the 64-cavity sweep the graph took the FP64
@@ -613,6 +627,21 @@ class DeviceSystem {
             const char *ea = std::getenv("HFH_AMG");
             k64.want_amg = k32.want_amg = amg && !(ea && std::strcmp(ea, "0") == 0);
             k64.amg_max_cx = k32.amg_max_cx = amg_max_cx;
+        }
+        // matrices with a Kronecker form are solved directly; their hierarchy
+        // is built when a solve or a probe first needs it
+        {
+            std::vector<int> so = seg_off;
+            fdm.ready = fdm_allowed() && fdm.build(hrp, hci, hv, so, st);
+        }
+        k64.defer_amg = k32.defer_amg = fdm.ready && k64.want_amg;
+        hrp_.clear();
+        hci_.clear();
+        hv_.clear();
+        if (k64.defer_amg) {
+            hrp_ = hrp;
+            hci_ = hci;
+            hv_ = hv;
         }
         t_mixed_ = t_fp64_ = -1;
         n32_ = n64_ = 0;
@@ -702,14 +731,87 @@ class DeviceSystem {
         return used;
     }
 
+    // A run that names a form of the Krylov or V-cycle kernels by one of
+    // their switches gets these kernels; HFH_FDM=0 turns the direct solves off
+    static bool fdm_allowed() {
+        if (const char *e = std::getenv("HFH_FDM"))
+            if (std::strcmp(e, "0") == 0) return false;
+        if (const char *e = std::getenv("HFH_MIXED_FP32"))
+            if (std::strcmp(e, "1") == 0) return false;
+        for (const char *k : {"HFH_KRYLOV", "HFH_KRYLOV_LANES", "HFH_KRYLOV_ROWS", "HFH_KRYLOV_TIMED_LANES", "HFH_AMG",
+                              "HFH_AMG_PCG", "HFH_AMG_FUSE", "HFH_AMG_OMEGA", "HFH_AMG_THETA", "HFH_AMG_LANES",
+                              "HFH_AMG_DIAG", "HFH_VEL_AMG", "HFH_MIXED_AMG32", "HFH_TEMPLATES", "HFH_DIAG",
+                              "HFH_GRAPH", "HFH_FIRST_PASS", "HFH_RESTARTS"})
+            if (std::getenv(k)) return false;
+        return true;
+    }
+    // builds the hierarchies that set_matrix deferred
+    void ensure_amg(hipStream_t st) {
+        if (hrp_.empty()) return;
+        k64.build_amg(hrp_, hci_, hv_, st);
+        k32.build_amg(hrp_, hci_, hv_, st);
+        hrp_.clear();
+        hci_.clear();
+        hv_.clear();
+    }
+
+    // Direct solve (hfh_fdm.hpp): x += M (b - A x) until the true residual
+    // passes the stopping test or stops falling.  False when the corrections
+    // do not converge (the caller goes on with the Krylov solver from x).
+    bool fdm_solve(const double *b, double *x, double rtol, double atol, hipStream_t st, SolveStats &S) {
+        const double *h = reinterpret_cast<const double *>(hpin_ + off_fd_);
+        std::vector<SolveStats> gs(nseg);
+        double best = -1.0;
+        true_residual(x, b, st);
+        for (int pass = 1; pass <= 4; pass++) {
+            if (pass > 1) HFH_CHECK(hipMemcpyAsync(xbak.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
+            fdm.correct(r.p, x, part3.p, dinv.p, st);
+            true_residual(x, b, st);
+            k_fdm_norms<<<nseg, 256, 0, st>>>(fdm.w0.p, part1.p, part2.p, reinterpret_cast<double *>(hpin_ + off_fd_));
+            HFH_CHECK(hipStreamSynchronize(st));
+            bool all_conv = true;
+            double worst = 0;
+            for (int g = 0; g < nseg; g++) {
+                const double rn = std::sqrt(h[2 * g]), bn = std::sqrt(h[2 * g + 1]), tol = std::max(rtol * bn, atol);
+                gs[g].iters = pass;
+                gs[g].resid = bn > 0 ? rn / bn : rn;
+                gs[g].converged = rn <= tol;
+                all_conv = all_conv && gs[g].converged;
+                worst = std::isfinite(gs[g].resid) ? std::max(worst, gs[g].resid) : gs[g].resid;
+                if (!std::isfinite(worst)) break;
+            }
+            S.iters = pass;
+            if (!std::isfinite(worst)) {
+                all_conv = false;
+                if (pass == 1) return false;
+            }
+            const bool better = pass == 1 || worst < best;
+            if (!better) {
+                HFH_CHECK(hipMemcpyAsync(x, xbak.p, n * sizeof(double), hipMemcpyDeviceToDevice, st));
+            } else {
+                seg_stats = gs;
+                S.resid = worst;
+                S.converged = all_conv;
+            }
+            if (all_conv) return true;
+            // a correction that no longer halves the residual has reached its
+            // rounding (b - A x carries eps |A| |x|)
+            if (pass > 1 && !(worst < 0.5 * best)) break;
+            best = worst;
+        }
+        // at the rounding of the residual the Krylov solver has nothing to add
+        return S.resid < 1e-8;
+    }
+
     // r = b - A x and the per-256-row partials of r.r and b.b in part1 /
     // part2: the diagonal-form rows when the FP64 solver has them
     // (HFH_RESID_DIAG=0: the CSR launch)
     void true_residual(const double *x, const double *b, hipStream_t st) {
         if (k64.Av.dw && resid_diag_)
-            k_residual_d<double><<<(n + KNT - 1) / KNT, KNT, 0, st>>>(n, k64.Av, x, b, r.p, part1.p, part2.p, nb);
+            k_residual_d<double><<<(n + KNT - 1) / KNT, KNT, 0, st>>>(n, k64.Av, x, b, r.p, part1.p, part2.p,
+                                                                       part3.p, nb);
         else
-            k_residual_l4<double><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p);
+            k_residual_l4<double><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p);
     }
 
     // FP64 fused solve: Jacobi-PCG (spd) or BiCGStab, warm-started from x.
@@ -717,6 +819,12 @@ class DeviceSystem {
     // passes, the true residual b - A x is checked and the iteration
     // restarted from x (at most twice) while it misses the tolerance.
     SolveStats fused64(bool spd, const double *b, double *x, double rtol, double atol, int maxit, hipStream_t st) {
+        if (fdm.ready && maxit > 0) {
+            SolveStats F;
+            if (fdm_solve(b, x, rtol, atol, st, F)) return F;
+            fdm.ready = false;
+        }
+        ensure_amg(st);
         int hi[KI_N];
         double hs[KS_N];
         SolveStats S;
@@ -874,6 +982,16 @@ class DeviceSystem {
     // all segments together, each against its own tolerance.
     SolveStats fused_mixed(bool spd, const double *b, double *x, double rtol, double atol, double inner_rtol,
                            int maxit, hipStream_t st) {
+        if (fdm.ready && maxit > 0) {
+            SolveStats F;
+            if (fdm_solve(b, x, rtol, atol, st, F)) {
+                F.fallback = 2;  // FP64 throughout
+                for (auto &g : seg_stats) g.fallback = 2;
+                return F;
+            }
+            fdm.ready = false;
+        }
+        ensure_amg(st);
         account_pending();
         bool use32, probing = false;
         const bool pref32 = t_mixed_ >= 0 && t_fp64_ >= 0 && t_mixed_ < t_fp64_;
@@ -1229,6 +1347,9 @@ class DeviceSystem {
   private:
     char *hpin_ = nullptr;  // pinned status: flags at 0, fused scalars at 64, outer scalars at 256
     int off_rr_ = 512;      // pinned true-residual partials (r.r then b.b, nb each)
+    int off_fd_ = 0;        // pinned r.r and b.b per segment (direct solves)
+    std::vector<int> hrp_, hci_;  // the matrix, while its hierarchy is deferred
+    std::vector<double> hv_;
     bool graph_on_ = false;  // first pass of FP64 fused solves as a captured graph (HFH_GRAPH=1)
     bool first_pass_ = false;  // one wait for flags and true residual (HFH_FIRST_PASS=1, or with graphs)
     bool resid_diag_ = true;  // true residuals through the diagonal-form rows (HFH_RESID_DIAG)
