@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(FDM_NT) k_fdm(const int4 *__restrict__ tiles, 
 
 // r.r and b.b of each segment from the 256-row partials, written to pinned
 // host memory (one workgroup per segment)
-__global__ void __launch_bounds__(256) k_fdm_norms(const int *__restrict__ w0, const double *__restrict__ prr,
+__global__ void __launch_bounds__(256) k_seg_norms(const int *__restrict__ w0, const double *__restrict__ prr,
                                                    const double *__restrict__ pbb, double *out) {
     __shared__ double s1[4], s2[4];
     double a = 0, b = 0;
@@ -425,13 +425,14 @@ class FdmSolver {
   public:
     bool ready = false;
     int n = 0, nd = 0, nsys = 0;
-    KBuf<int> w0;  // first 256-row block of each segment, and the end
 
     // segments as DeviceSystem::set_matrix takes them; false (no plan) when
-    // a segment has no Kronecker form
+    // a segment has no Kronecker form, or no coupling reaches min_coupling
+    // of the diagonal
     bool build(const std::vector<int> &rp, const std::vector<int> &ci, const std::vector<double> &v,
-               const std::vector<int> &seg, hipStream_t st) {
+               const std::vector<int> &seg, hipStream_t st, double min_coupling = 0) {
         ready = false;
+        double coupling = 0;
         n = (int)rp.size() - 1;
         nsys = (int)seg.size() - 1;
         if (n <= 0 || nsys <= 0) return false;
@@ -443,7 +444,9 @@ class FdmSolver {
             const int d = sy[q].n[2] > 1 ? 3 : 2;
             if (q > 0 && d != nd) return false;
             nd = d;
+            for (int e = 0; e < d; e++) coupling = std::max(coupling, std::fabs(sy[q].b[e]) / sy[q].a);
         }
+        if (coupling < min_coupling) return false;
         // the distinct one-dimensional matrices: V, then V^T
         std::map<std::tuple<int, int, int>, std::pair<long, std::vector<double>>> mat;
         std::vector<double> pool, lam;
@@ -465,7 +468,6 @@ class FdmSolver {
         std::vector<FdmJob> jobs;
         std::vector<FdmPin> pins(nsys);
         std::vector<std::vector<int4>> tl(2 * nd);
-        std::vector<int> hw(nsys + 1);
         bool pinned = false;
         for (int q = 0; q < nsys; q++) {
             const FdmSys &s = sy[q];
@@ -505,7 +507,7 @@ class FdmSolver {
             add(2 * nd - 1, ny * nz, nx, nx, nx, nx, nx, 1, 0, Z[0]);
             FdmPin &p = pins[q];
             p.off = s.off;
-            p.w0 = hw[q] = s.off / 256;
+            p.w0 = s.off / 256;
             p.w1 = (s.off + s.len + 255) / 256;
             if (s.pin >= 0) {
                 p.pin = s.pin;
@@ -518,7 +520,6 @@ class FdmSolver {
                 pinned = true;
             }
         }
-        hw[nsys] = (n + 255) / 256;
         for (int q = 0; q < 2 * nd; q++) {
             ntiles_[q] = (int)tl[q].size();
             put(tiles_[q], tl[q], st);
@@ -527,7 +528,6 @@ class FdmSolver {
         put(pins_, pins, st);
         put(mats_, pool, st);
         put(lam_, lam, st);
-        put(w0, hw, st);
         t0_.alloc(n);
         t1_.alloc(n);
         g_.alloc(n);

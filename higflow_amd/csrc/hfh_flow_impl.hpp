@@ -250,6 +250,22 @@ void Flow<D>::upload_device() {
     for (int d = 0; d < D; d++)
         if (!momRe_[d].empty()) dMomRe_[d].upload(momRe_[d].data(), momRe_[d].size(), st_);
     if (!vePar_.empty()) dVePar_.upload(vePar_.data(), vePar_.size(), st_);
+    // Factors of refined meshes (hfh_nd.hpp): for explicit runs, and for
+    // large semi-implicit runs in the mixed form, where they replace FP32
+    // refinements that end well below the tolerance.  FP64 iterations stop at
+    // the tolerance; the error they leave in u*, over dt, is 1e-9 of the
+    // pressure (3-level contraction, tolerance 1e-11, against runs at 1e-13),
+    // and semi-implicit runs whose systems are solved by them (all of the
+    // FP64 form, small ones of the mixed form) keep them and their results.
+    const bool semi = par_.tempdiscrtype == SEMI_IMPLICIT_EULER;
+    const bool factors = !semi || (par_.precision == 1 && Nc_ >= 65536);
+    psys_.nd_max_flops = hsysB_.nd_max_flops = factors ? 2e11 : 0;
+    // the same for nearly diagonal velocity systems of uniform meshes (no
+    // coupling at the strength threshold, so no hierarchy either), which
+    // converge in 2-7 Jacobi-PCG iterations: at a coupling of 0.05 and
+    // Re = 160 the direct solve moved the pressure by 2e-9, at 0.09 and above
+    // by 2.4e-10 at most
+    hsysB_.fdm_min_coupling = 0.08;
     psys_.set_matrix(Arp_, Aci_, Av_, st_, true, pseg_);
     if (par_.tempdiscrtype == SEMI_IMPLICIT_EULER) {
         const char *ek = std::getenv("HFH_KRYLOV");

@@ -26,6 +26,7 @@
 #include "hfh_kernels.hpp"
 #include "hfh_fused.hpp"
 #include "hfh_fdm.hpp"
+#include "hfh_nd.hpp"
 
 #define HFH_CHECK(x)                                                                        \
     do {                                                                                    \
@@ -510,6 +511,13 @@ class DeviceSystem {
     FusedKrylov<double> k64;
     FusedKrylov<float> k32;
     FdmSolver fdm;  // direct solves of Kronecker-sum matrices
+    NdSolver nd;    // and of other matrices whose factors are affordable
+    // operations that the set-up may spend on the factors of one matrix (0:
+    // none); a 16-core host takes about 2 s for 2e11
+    double nd_max_flops = 0;
+    // the direct solve wants a coupling of at least this share of the diagonal
+    double fdm_min_coupling = 0;
+    bool direct() const { return fdm.ready || nd.ready; }
     bool fused = true;
     int max_restarts = 1;      // fused64: restarts on the true residual
     double t_mixed_ = -1, t_fp64_ = -1;  // mixed form: seconds per solve of each form
@@ -533,6 +541,7 @@ class DeviceSystem {
     bool force32_ = false;  // HFH_MIXED_FP32=1: always refine with FP32 solves
     bool mixed_amg32_ = true;  // the mixed form's FP64 solves use the FP32 V-cycle
     int pred32_[3] = {0, 0, 0};  // FP32 iterations of the 1st, 2nd, later corrections
+    DevBuf<int> segw_;              // first 256-row block of each segment, and the end
     DevBuf<int> bseg_;              // segment of each BLOCK-row block (nseg > 1)
     DevBuf<double> segsc_;          // per-segment scale s_g and unscale u_g
     std::vector<double> hsegsc_;
@@ -612,6 +621,12 @@ class DeviceSystem {
             hpin_size_ = pin;
         }
         seg_stats.assign(nseg, SolveStats());
+        {
+            std::vector<int> hw(nseg + 1, (n + 255) / 256);
+            for (int g = 0; g < nseg; g++) hw[g] = seg_off[g] / 256;
+            segw_.upload(hw.data(), hw.size(), st);
+            HFH_CHECK(hipStreamSynchronize(st));  // hw is a local
+        }
         if (nseg > 1) {
             std::vector<int> hb(nb, nseg - 1);
             for (int g = 0; g < nseg; g++)
@@ -632,9 +647,16 @@ class DeviceSystem {
         // is built when a solve or a probe first needs it
         {
             std::vector<int> so = seg_off;
-            fdm.ready = fdm_allowed() && fdm.build(hrp, hci, hv, so, st);
+            const bool on = direct_allowed();
+            fdm.ready = on && fdm.build(hrp, hci, hv, so, st, fdm_min_coupling);
+            nd.ready = on && !fdm.ready && nd_max_flops > 0 && nd.build(hrp, hci, hv, st, nd_max_flops, 2.5e8);
+            if (const char *ev = std::getenv("HFH_VERBOSE"))
+                if (std::strcmp(ev, "1") == 0 && (nd_max_flops > 0 || fdm.ready))
+                    std::fprintf(stderr, "hfh: system of %d rows: %s (factors %.2g operations, %.2g entries)\n", n,
+                                 fdm.ready ? "fast diagonalisation" : nd.ready ? "nested dissection" : "Krylov",
+                                 nd.flops, nd.entries);
         }
-        k64.defer_amg = k32.defer_amg = fdm.ready && k64.want_amg;
+        k64.defer_amg = k32.defer_amg = direct() && k64.want_amg;
         hrp_.clear();
         hci_.clear();
         hv_.clear();
@@ -732,9 +754,9 @@ class DeviceSystem {
     }
 
     // A run that names a form of the Krylov or V-cycle kernels by one of
-    // their switches gets these kernels; HFH_FDM=0 turns the direct solves off
-    static bool fdm_allowed() {
-        if (const char *e = std::getenv("HFH_FDM"))
+    // their switches gets these kernels; HFH_DIRECT=0 turns the direct solves off
+    static bool direct_allowed() {
+        if (const char *e = std::getenv("HFH_DIRECT"))
             if (std::strcmp(e, "0") == 0) return false;
         if (const char *e = std::getenv("HFH_MIXED_FP32"))
             if (std::strcmp(e, "1") == 0) return false;
@@ -755,19 +777,22 @@ class DeviceSystem {
         hv_.clear();
     }
 
-    // Direct solve (hfh_fdm.hpp): x += M (b - A x) until the true residual
+    // Direct solve (hfh_fdm.hpp, hfh_nd.hpp): x += M (b - A x) until the true residual
     // passes the stopping test or stops falling.  False when the corrections
     // do not converge (the caller goes on with the Krylov solver from x).
-    bool fdm_solve(const double *b, double *x, double rtol, double atol, hipStream_t st, SolveStats &S) {
+    bool direct_solve(const double *b, double *x, double rtol, double atol, hipStream_t st, SolveStats &S) {
         const double *h = reinterpret_cast<const double *>(hpin_ + off_fd_);
         std::vector<SolveStats> gs(nseg);
         double best = -1.0;
         true_residual(x, b, st);
         for (int pass = 1; pass <= 4; pass++) {
             if (pass > 1) HFH_CHECK(hipMemcpyAsync(xbak.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
-            fdm.correct(r.p, x, part3.p, dinv.p, st);
+            if (fdm.ready)
+                fdm.correct(r.p, x, part3.p, dinv.p, st);
+            else
+                nd.correct(r.p, x, st);
             true_residual(x, b, st);
-            k_fdm_norms<<<nseg, 256, 0, st>>>(fdm.w0.p, part1.p, part2.p, reinterpret_cast<double *>(hpin_ + off_fd_));
+            k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part2.p, reinterpret_cast<double *>(hpin_ + off_fd_));
             HFH_CHECK(hipStreamSynchronize(st));
             bool all_conv = true;
             double worst = 0;
@@ -819,10 +844,10 @@ class DeviceSystem {
     // passes, the true residual b - A x is checked and the iteration
     // restarted from x (at most twice) while it misses the tolerance.
     SolveStats fused64(bool spd, const double *b, double *x, double rtol, double atol, int maxit, hipStream_t st) {
-        if (fdm.ready && maxit > 0) {
+        if (direct() && maxit > 0) {
             SolveStats F;
-            if (fdm_solve(b, x, rtol, atol, st, F)) return F;
-            fdm.ready = false;
+            if (direct_solve(b, x, rtol, atol, st, F)) return F;
+            fdm.ready = nd.ready = false;
         }
         ensure_amg(st);
         int hi[KI_N];
@@ -982,14 +1007,14 @@ class DeviceSystem {
     // all segments together, each against its own tolerance.
     SolveStats fused_mixed(bool spd, const double *b, double *x, double rtol, double atol, double inner_rtol,
                            int maxit, hipStream_t st) {
-        if (fdm.ready && maxit > 0) {
+        if (direct() && maxit > 0) {
             SolveStats F;
-            if (fdm_solve(b, x, rtol, atol, st, F)) {
+            if (direct_solve(b, x, rtol, atol, st, F)) {
                 F.fallback = 2;  // FP64 throughout
                 for (auto &g : seg_stats) g.fallback = 2;
                 return F;
             }
-            fdm.ready = false;
+            fdm.ready = nd.ready = false;
         }
         ensure_amg(st);
         account_pending();
