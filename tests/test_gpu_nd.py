@@ -60,8 +60,10 @@ def test_pressure_of_a_refined_mesh(which, monkeypatch):
 def test_velocity_blocks_of_a_large_mixed_run(monkeypatch):
     case = cases.contraction(levels=4, graded=True, h0=0.05, dt=1e-5, rtol=RTOL, atol=0.0, maxit=50000)
     a, b = _pair(case, monkeypatch, precision=1, inner_rtol=1e-5)
-    for d in range(2):
-        sa, sb = a.solve_stats(1 + d), b.solve_stats(1 + d)
-        assert sa["iters"] <= 4 < sb["iters"] and sa["resid"] <= max(RTOL, sb["resid"])
-        x, y = a.get(3, d), b.get(3, d)
-        assert np.linalg.norm(x - y) <= _cond(a, 1 + d) * (sa["resid"] + sb["resid"]) * np.linalg.norm(y)
+    # the component that the inflow drives (the other's right-hand side is
+    # zero at rest)
+    sa, sb = a.solve_stats(1), b.solve_stats(1)
+    assert sa["iters"] <= 4 < sb["iters"] and sa["resid"] <= max(RTOL, sb["resid"])
+    x, y = a.get(3, 0), b.get(3, 0)
+    assert np.linalg.norm(x - y) <= _cond(a, 1) * (sa["resid"] + sb["resid"]) * np.linalg.norm(y)
+    assert not a.get(3, 1).any() and not b.get(3, 1).any()
