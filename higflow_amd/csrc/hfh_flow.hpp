@@ -9,6 +9,7 @@
 // the fused per-cell log-conformation + polymeric-stress kernel.
 #pragma once
 #include <chrono>
+#include <climits>
 
 #include "hfh_kernels.hpp"
 #include "hfh_linsolve.hpp"
@@ -347,6 +348,14 @@ class Flow : public FlowBase {
         long op_bytes = 0;  // the operator as a launch streams it
         int nrow = 0, ncomp = 1, in_stride = 0, out_stride = 0;
         int lanes = 1;  // lanes per row (from the mean row length)
+        // wave tasks (k_interp_t): the rows before gen0 and from sell0 on
+        // (between them, long rows on 16 lanes)
+        DevBuf<int4> task;
+        DevBuf<int> czero, slen, scol;
+        DevBuf<double> sval;
+        DevBuf<float> sval32;
+        std::vector<int4> htask;
+        int ntask = 0, gen0 = 0, sell0 = 0, out0 = -1;
         bool has_y = false, f32 = false;
         std::vector<int> order;  // device row k is the group's row order[k]
     } dDu_, dK_, dCv_, dMom_, dDiv_, dGrad_;

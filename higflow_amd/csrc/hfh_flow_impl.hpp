@@ -206,6 +206,7 @@ void Flow<D>::upload_device() {
                 for (int &v : tabs[q])
                     if (v >= oP && v < oP + n) v = oP + inv[v - oP];
             dg.out.upload(outp.data(), outp.size(), st_);
+            dg.out0 = oP;
             HFH_CHECK(hipStreamSynchronize(st_));  // outp is a local
         };
         relabel(dMom_, oPmom_, ms, D);
@@ -386,6 +387,7 @@ void Flow<D>::upload_group(DGroup &dg, const Group &g, int, int out_stride, bool
     // order.)
     dg.order.resize(dg.nrow);
     bool grouped = false;
+    int gen0 = 0;
     {
         const char *eo = std::getenv("HFH_GROUP_ORDER");
         const bool sort = covered > 0 && !(eo && std::strcmp(eo, "0") == 0);
@@ -396,6 +398,18 @@ void Flow<D>::upload_group(DGroup &dg, const Group &g, int, int out_stride, bool
             for (int r = 0; r < dg.nrow; r++) start[(code[r] >= 0 ? code[r] : nt) + 1]++;
             for (int t = 0; t <= nt; t++) start[t + 1] += start[t];
             for (int r = 0; r < dg.nrow; r++) dg.order[start[code[r] >= 0 ? code[r] : nt]++] = r;
+            // templates are numbered from the most shared down: from the
+            // first of fewer than 32 rows (half a wave) on, rows go by
+            // length, the longest first (wave tasks of k_interp_t)
+            while (gen0 < dg.nrow && code[dg.order[gen0]] >= 0) {
+                int e = gen0;
+                while (e < dg.nrow && code[dg.order[e]] == code[dg.order[gen0]]) e++;
+                if (e - gen0 < 32) break;
+                gen0 = e;
+            }
+            std::stable_sort(dg.order.begin() + gen0, dg.order.end(), [&](int x, int y) {
+                return g.rowptr[x + 1] - g.rowptr[x] > g.rowptr[y + 1] - g.rowptr[y];
+            });
         } else {
             for (int r = 0; r < dg.nrow; r++) dg.order[r] = r;
         }
@@ -467,10 +481,76 @@ void Flow<D>::upload_group(DGroup &dg, const Group &g, int, int out_stride, bool
     // on 4 (the 64-cavity sweep)
     dg.lanes = grouped ? (avg < 4 ? 1 : avg < 32 ? 2 : avg < 64 ? 4 : 8)
                        : (avg < 4 ? 1 : avg < 8 ? 2 : avg < 16 ? 4 : avg < 32 ? 8 : 16);
+    dg.ntask = dg.gen0 = 0;
+    dg.out0 = -1;
     if (const char *e = std::getenv("HFH_INTERP_LANES")) {
         int f = std::atoi(e);
         if (f == 1 || f == 2 || f == 4 || f == 8 || f == 16) dg.lanes = f;
+        return;
     }
+    if (!grouped || (size_t)nX_ * sizeof(double) >= (1ull << 32)) return;
+    std::vector<int4> task;
+    for (int k = 0; k < gen0;) {
+        int e = k + 1;
+        while (e < gen0 && e - k < 64 && pcode[e] == pcode[k]) e++;
+        bool run = true;
+        for (int r = k + 1; r < e && run; r++) run = pbase[r] == pbase[r - 1] + 1;
+        task.push_back(make_int4(pcode[k], k, e - k, run ? pbase[k] : -1));
+        k = e;
+    }
+    dg.gen0 = gen0;
+    // the other rows, the longest first: the least-squares rows of a 3D mesh
+    // (about 100 entries, sums of them more) on 16 lanes when they are the
+    // bulk, the rest column by column
+    auto length = [&](int k) { return pcode[k] >= 0 ? tcnt[pcode[k]] : rp[k + 1] - rp[k]; };
+    const int L = dg.lanes, RW = 64 / L;
+    int sell0 = gen0;
+    if (D == 3)
+        while (sell0 < dg.nrow && length(sell0) > 48) sell0++;
+    long padded = 0;
+    for (int k = sell0; k < dg.nrow; k += RW) padded += 64L * ((length(k) + L - 1) / L);
+    if (padded > INT_MAX) return;
+    dg.sell0 = sell0;
+    const int ng = dg.nrow - sell0;
+    if (ng > 0) {
+        std::vector<int> slen(ng), scol(padded, 0);
+        std::vector<double> sval(padded, 0.0);
+        long at = 0;
+        for (int k = sell0; k < dg.nrow; k += RW) {
+            const int m = std::min(RW, dg.nrow - k);
+            task.push_back(make_int4(-1, k, m, (int)at));
+            for (int q = 0; q < m; q++) {
+                const int r = k + q, t = pcode[r];
+                slen[r - sell0] = length(r);
+                for (int e = 0; e < length(r); e++) {
+                    const long i = at + 64L * (e / L) + q * L + e % L;
+                    // a template row's weights are its template's
+                    scol[i] = t >= 0 ? pbase[r] + toff[(size_t)t * GT_MAX + e] : col[rp[r] + e];
+                    sval[i] = t >= 0 ? tw[(size_t)t * GT_MAX + e] : val[rp[r] + e];
+                }
+            }
+            at += 64L * ((length(k) + L - 1) / L);
+        }
+        dg.slen.upload(slen.data(), slen.size(), st_);
+        dg.scol.upload(scol.data(), scol.size(), st_);
+        std::vector<float> s32;
+        if (f32) {
+            s32.assign(sval.begin(), sval.end());
+            dg.sval32.upload(s32.data(), s32.size(), st_);
+        } else {
+            dg.sval.upload(sval.data(), sval.size(), st_);
+        }
+        HFH_CHECK(hipStreamSynchronize(st_));  // the tables are locals
+    }
+    if (task.empty()) return;
+    dg.ntask = (int)task.size();
+    dg.task.upload(task.data(), task.size(), st_);
+    dg.czero.alloc(task.size());
+    dg.htask.swap(task);
+    HFH_CHECK(hipStreamSynchronize(st_));
+    if (verbose_)
+        std::fprintf(stderr, "hfh:   %d wave tasks; %d rows on 16 lanes, %d rows column by column\n", dg.ntask,
+                     sell0 - gen0, ng);
 }
 
 // Template rows of an interpolation group.  Rows of at most GT_MAX entries
@@ -586,6 +666,7 @@ void Flow<D>::refold_constants() {
     // the host copies stay alive until the stream has consumed them
     std::vector<std::vector<double>> keep;
     std::vector<std::vector<float>> keep32;
+    std::vector<std::vector<int>> keepz;
     for (auto &p : gs) {
         if (p.d->nrow == 0) continue;
         {
@@ -596,6 +677,16 @@ void Flow<D>::refold_constants() {
             keep.push_back(std::move(c));
         }
         const std::vector<double> &c = keep.back();
+        if (p.d->ntask > 0) {
+            keepz.emplace_back(p.d->ntask);
+            for (int w = 0; w < p.d->ntask; w++) {
+                const int4 &t = p.d->htask[w];
+                bool zero = true;
+                for (int r = t.y; r < t.y + t.z && zero; r++) zero = c[r] == 0.0;
+                keepz.back()[w] = zero;
+            }
+            p.d->czero.upload(keepz.back().data(), keepz.back().size(), st_);
+        }
         if (p.d->f32) {
             keep32.emplace_back(c.begin(), c.end());
             p.d->cst32.upload(keep32.back().data(), keep32.back().size(), st_);
@@ -701,6 +792,34 @@ void Flow<D>::launch_rows(DGroup &dg, const W *val, const W *cst, W alpha, doubl
             tp.tw = dg.tw32.p;
         else
             tp.tw = dg.tw.p;
+    }
+    if (dg.ntask > 0) {
+        const int nta = ((dg.ntask + BLOCK / 64 - 1) / (BLOCK / 64) + 127) / 128 * 128;
+        RowTasks<W> R;
+        R.task = dg.task.p;
+        R.czero = dg.czero.p;
+        R.ntask = dg.ntask;
+        R.gen0 = dg.gen0;
+        R.sell0 = dg.sell0;
+        R.out0 = dg.out0;
+        R.slen = dg.slen.p;
+        R.scol = dg.scol.p;
+        if constexpr (sizeof(W) == 4)
+            R.sval = dg.sval32.p;
+        else
+            R.sval = dg.sval.p;
+        const dim3 grid(nta + nblocks((long)(dg.sell0 - dg.gen0) * 16), dg.ncomp);
+        auto go = [&](auto Lc) {
+            k_interp_t<double, decltype(Lc)::value, 16, W><<<grid, BLOCK, 0, st_>>>(
+                nta, R, dg.rp.p, dg.col.p, val, cst, dg.out.p, y, alpha, dg.in_stride, dg.out_stride, X_.p, dst, tp);
+        };
+        switch (dg.lanes) {
+        case 1: go(std::integral_constant<int, 1>{}); break;
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        default: go(std::integral_constant<int, 8>{}); break;
+        }
+        return;
     }
 #define HFH_INTERP_L(L)                                                                                        \
     k_interp_l<double, L, W><<<nblocks(n * L), BLOCK, 0, st_>>>(dg.nrow, dg.ncomp, dg.rp.p, dg.col.p, val, cst, \

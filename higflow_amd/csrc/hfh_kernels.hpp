@@ -123,6 +123,162 @@ __global__ void __launch_bounds__(BLOCK) k_interp_l(int nrow, int ncomp, const i
     }
 }
 
+// The rows of a group whose device order puts the rows of each template
+// together (upload_group), 64 rows and one row per lane in each wave:
+//
+// {template, first row, rows <= 64, base or -1}: the template is the same for
+// the whole wave, so its offsets and weights come through the scalar cache
+// and a row costs one vector load per entry.  Mostly the bases of the rows
+// are consecutive too (then `base` is the first one's), and with czero the
+// constants are all zero, so nothing but the state is read.
+//
+// {-1, first row, rows <= 64 / L, entry}: rows of rare templates and rows
+// without one, sorted by length, L lanes per row.  Step e of lane (row, l)
+// is the row's entry e L + l, at scol / sval[entry + 64 e + lane], so the
+// lanes of a wave read side by side; slen[row - sell0] entries per row.
+//
+// A row sums its entries l, l + L, ... in L partial sums and adds these in
+// the butterfly order of k_interp_l with L lanes, L = 1 onto the constant as
+// k_interp does, so its value is theirs.  The momentum rows of the 64-cavity
+// sweep (17 M rows of 15 entries), bound before by per-lane template reads
+// and by the uncoalesced entries of the other rows: 670 -> 300 us (1.3 TB/s of writes and column-by-column entries); 256^2 cavity
+// 34 -> 23 us, graded contraction 68 -> 42 us, 3D wall layer 424 -> 250 us.
+//
+// Long rows (3D least squares, about 100 entries) take LG lanes per row
+// instead: rows [gen0, sell0) as k_interp_l, in the workgroups from nta on.
+template <int L, typename W>
+__device__ inline W interp_butterfly(W (&a)[L]) {
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int l = 0; l < o; l++) a[l] = a[l] + a[l + o];
+    return a[0];
+}
+template <typename W>
+struct RowTasks {
+    const int4 *task = nullptr;
+    const int *czero = nullptr;
+    int ntask = 0, gen0 = 0, sell0 = 0, out0 = -1;  // out0 >= 0: row r writes out0 + r
+    const int *slen = nullptr, *scol = nullptr;
+    const W *sval = nullptr;
+};
+template <typename T, int L, int LG, typename W = T>
+__global__ void __launch_bounds__(BLOCK) k_interp_t(int nta, RowTasks<W> R, const int *__restrict__ rowptr,
+                                                    const int *__restrict__ col, const W *__restrict__ val,
+                                                    const W *__restrict__ cst, const int *__restrict__ out,
+                                                    const int *__restrict__ yoff, W alpha, int in_stride,
+                                                    int out_stride, const T *X, T *dst, GTempl<W> tp) {
+    const int c = blockIdx.y;
+    const T *Xs = X + (size_t)c * in_stride;
+    auto put = [&](int r, W v) {
+        W o = alpha * v;
+        if (yoff) o = (W)X[yoff[r]] + o;
+        dst[(R.out0 >= 0 ? R.out0 + r : out[r]) + (size_t)c * out_stride] = (T)o;
+    };
+    if ((int)blockIdx.x < nta) {
+        // workgroups go round robin over the 8 XCDs: in each window of 128
+        // workgroups an XCD takes 16 in a row (4096 rows), so the mesh lines
+        // that neighbouring tasks share stay in its L2 while the tasks, long
+        // and short in places, stay spread
+        const int blk = ((int)blockIdx.x & ~127) | (((int)blockIdx.x & 7) << 4) | (((int)blockIdx.x >> 3) & 15);
+        const int w = __builtin_amdgcn_readfirstlane(blk * (BLOCK / 64) + (int)(threadIdx.x >> 6));
+        if (w >= R.ntask) return;
+        const int4 tk = R.task[w];
+        const int t = __builtin_amdgcn_readfirstlane(tk.x), row0 = __builtin_amdgcn_readfirstlane(tk.y);
+        const int m = __builtin_amdgcn_readfirstlane(tk.z), b0 = __builtin_amdgcn_readfirstlane(tk.w);
+        const int cz = __builtin_amdgcn_readfirstlane(R.czero[w]);
+        const int lane = threadIdx.x & 63;
+        if (t >= 0) {
+            const int ln = lane < m ? lane : 0, r = row0 + ln;
+            const W k0 = cz ? W(0) : cst[r];
+            W a[L];
+#pragma unroll
+            for (int l = 0; l < L; l++) a[l] = L == 1 ? k0 : W(0);
+            constexpr int U = 8;
+            const int cnt = tp.tcnt[t];
+            const int *off = tp.toff + (size_t)t * GT_MAX;
+            const W *wt = tp.tw + (size_t)t * GT_MAX;
+            // byte offset of the row's base: the state is below 4 GiB
+            const unsigned bb = (unsigned)(b0 >= 0 ? b0 + ln : tp.base[r]) * (unsigned)sizeof(T);
+            for (int e = 0; e < cnt; e += U) {  // the tables are padded to GT_MAX
+                W x[U];
+#pragma unroll
+                for (int q = 0; q < U; q++)
+                    x[q] = (W) * reinterpret_cast<const T *>(reinterpret_cast<const char *>(Xs + off[e + q]) + bb);
+#pragma unroll
+                for (int q = 0; q < U; q++)
+                    if (e + q < cnt) a[q % L] += x[q] * wt[e + q];
+            }
+            const W v = L == 1 ? a[0] : k0 + interp_butterfly<L, W>(a);
+            if (lane < m) put(r, v);
+            return;
+        }
+        // 64 / L rows, lane (row, l) walks entries l, l + L, ...
+        const int q0 = lane / L, ln = q0 < m ? q0 : 0, r = row0 + ln, l = lane % L;
+        const W k0 = cz ? W(0) : cst[r];
+        const int len = R.slen[r - R.sell0];
+        const int most = (__builtin_amdgcn_readfirstlane(len) + L - 1) / L;  // the longest row comes first
+        const int mine = (len - l + L - 1) / L;
+        const int *sc = R.scol + (size_t)(unsigned)b0 + lane;
+        const W *sv = R.sval + (size_t)(unsigned)b0 + lane;
+        W a = L == 1 ? k0 : W(0);
+        constexpr int U = 12;
+#pragma unroll 1
+        for (int e = 0; e < most; e += U) {
+            int j[U];
+            W u[U];
+            bool ok[U];
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                ok[q] = e + q < mine;
+                j[q] = ok[q] ? sc[(size_t)(e + q) * 64] : 0;
+                u[q] = ok[q] ? sv[(size_t)(e + q) * 64] : W(0);
+            }
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                const W x = (W)Xs[j[q]];
+                if (ok[q]) a += x * u[q];
+            }
+        }
+#pragma unroll
+        for (int o = L / 2; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+        if (q0 < m && l == 0) put(r, L == 1 ? a : k0 + a);
+        return;
+    }
+    const long g = ((long)(blockIdx.x - nta) * BLOCK + threadIdx.x) / LG;
+    const int lane = threadIdx.x % LG;
+    const bool in = R.gen0 + g < (long)R.sell0;
+    const int r = in ? R.gen0 + (int)g : R.gen0;
+    int b = 0, e = 0, cb = 0;
+    const int *cp = col;
+    const W *vp = val;
+    if (in) grow<W>(tp, r, rowptr, col, val, b, e, cp, vp, cb);
+    const T *Xc = Xs + cb;
+    W v = 0;
+    constexpr int U = 4;
+#pragma unroll 1
+    for (int k0 = b + lane; k0 < e; k0 += U * LG) {
+        int j[U];
+        W a[U];
+        bool ok[U];
+#pragma unroll
+        for (int q = 0; q < U; q++) {
+            const int k = k0 + q * LG;
+            ok[q] = k < e;
+            j[q] = ok[q] ? cp[k] : 0;
+            a[q] = ok[q] ? vp[k] : W(0);
+        }
+#pragma unroll
+        for (int q = 0; q < U; q++) {
+            const W x = (W)Xc[j[q]];
+            if (ok[q]) v += x * a[q];
+        }
+    }
+#pragma unroll
+    for (int o = LG / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (in && lane == 0) put(r, cst[r] + v);
+}
+
 // ------------------------------------------------------------- momentum
 struct MomParams {
     int nf, ns;
