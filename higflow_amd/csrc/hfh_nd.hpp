@@ -13,8 +13,8 @@
 // with W = F21 inv(F11), U = inv(F11) F12 of each front.
 //
 // Measured on MI355X (20 steps; 10 in 3D), against AMG-BiCGStab and FP32
-// refinement: graded 4-level contraction, mixed form, 226 -> 30 ms;
-// 12^3 wall-layer cavity 57 -> 13 ms, where a solve reads 0.57 GB of factors
+// refinement: graded 4-level contraction, mixed form, 226 -> 19 ms;
+// 12^3 wall-layer cavity 56 -> 7.3 ms, where a solve reads 0.57 GB of factors
 // (host factors: 1.5e11 operations, 4 s on 8 cores).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -419,87 +419,123 @@ class NdTree {
 };
 
 // ---------------------------------------------------------------- device
-struct NdDev {
-    int p, q;        // pivots, border
-    int po, bo;      // first pivot / border entry of the node's lists
-    int kid0, kid1;  // children
-    long w, g;       // W and G in the factor array
+// One workgroup's share of a front: rows [row0, row1) of W (up) or of
+// G = [inv(F11) | -U] (down), one row per lane group.  Everything that the
+// workgroup needs to find its data is here, so it starts its matrix loads
+// one memory round trip after the launch.
+struct NdTask {
+    int row0, row1;
+    int p, q;     // pivots, border
+    int po, bo;   // first pivot / border entry of the node's lists
+    int fo;       // first front entry (gather lists of the up pass)
+    int gl;       // lanes per row
+    long at;      // W or G in the factor array
 };
 constexpr int ND_NT = 256;
 constexpr int ND_LDS = 8192;  // front entries held in LDS (64 KiB)
+constexpr int ND_PRE = 16;    // matrix entries per lane in flight before the gather
+// lanes per row: enough that the whole row is in flight (up to 1024 entries)
+inline int nd_lanes(int len) { return len <= 8 * ND_PRE ? 8 : len <= 16 * ND_PRE ? 16 : 64; }
 
-// rows [row0, row1) of dot products with the vector v (len entries, LDS),
-// GL lanes per row; f(row, sum) on the group's first lane.  Four loads per
-// lane are in flight.
-template <int GL, typename F>
-__device__ inline void nd_rows(const double *__restrict__ M, int len, int row0, int row1, const double *v, F &&f) {
-    const int lane = threadIdx.x % GL;
-    for (int r = row0 + (int)threadIdx.x / GL; r < row1; r += ND_NT / GL) {
-        const double *m = M + (size_t)r * len;
-        double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-        int k = lane;
-        for (; k + 3 * GL < len; k += 4 * GL) {
-            const double a0 = m[k], a1 = m[k + GL], a2 = m[k + 2 * GL], a3 = m[k + 3 * GL];
-            s0 += a0 * v[k];
-            s1 += a1 * v[k + GL];
-            s2 += a2 * v[k + 2 * GL];
-            s3 += a3 * v[k + 3 * GL];
-        }
-        for (; k < len; k += GL) s0 += m[k] * v[k];
-        double s = (s0 + s1) + (s2 + s3);
+// The rows' matrix loads are issued first, then gather() fills the vector in
+// LDS (dependent index loads), then the dot products: the two chains of
+// memory round trips overlap.  A height of a few fronts is bound by this
+// latency (11-19 us with the loads behind the gather and the rows of a wave
+// in turn, 5-8 us so), the leaves by the factor bytes (250 MB in 37 us).
+template <int GL, typename Gather, typename Put>
+__device__ inline void nd_rows(const NdTask &T, const double *__restrict__ fac, int len, const double *v, Gather &&gather,
+                               Put &&put) {
+    const int row = T.row0 + (int)threadIdx.x / GL, lane = threadIdx.x % GL;
+    const bool in = row < T.row1;
+    const double *m = fac + T.at + (size_t)(in ? row : T.row0) * len;
+    double a[ND_PRE];
 #pragma unroll
-        for (int o = GL / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-        if (lane == 0) f(r, s);
-    }
+    for (int q = 0; q < ND_PRE; q++) a[q] = in && lane + q * GL < len ? m[lane + q * GL] : 0.0;
+    gather();
+    __syncthreads();
+    double s[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < ND_PRE; q++)
+        if (lane + q * GL < len) s[q & 3] += a[q] * v[lane + q * GL];
+    if (in)
+        for (int k = lane + ND_PRE * GL; k < len; k += ND_PRE * GL) {
+#pragma unroll
+            for (int q = 0; q < ND_PRE; q++) a[q] = k + q * GL < len ? m[k + q * GL] : 0.0;
+#pragma unroll
+            for (int q = 0; q < ND_PRE; q++)
+                if (k + q * GL < len) s[q & 3] += a[q] * v[k + q * GL];
+        }
+    double t = (s[0] + s[1]) + (s[2] + s[3]);
+#pragma unroll
+    for (int o = GL / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+    if (in && lane == 0) put(row, t);
+}
+template <typename Gather, typename Put>
+__device__ inline void nd_dispatch(const NdTask &T, const double *__restrict__ fac, int len, const double *v,
+                                   Gather &&gather, Put &&put) {
+    if (T.gl == 8)
+        nd_rows<8>(T, fac, len, v, gather, put);
+    else if (T.gl == 16)
+        nd_rows<16>(T, fac, len, v, gather, put);
+    else
+        nd_rows<64>(T, fac, len, v, gather, put);
 }
 
-// Up: one workgroup per (node, rows of W) of a tree height.  The front's
-// right-hand side is gathered into LDS (the children in turn, so no two
-// lanes add to one entry), then update = rhs_q - W rhs_p.
-__global__ void __launch_bounds__(ND_NT) k_nd_up(const int4 *__restrict__ tasks, const NdDev *__restrict__ nodes,
-                                                 const int *__restrict__ kids, const int *__restrict__ piv,
-                                                 const int *__restrict__ cmap, const double *__restrict__ fac,
-                                                 const double *__restrict__ r, double *__restrict__ y, double *upd) {
+// Up: the front's right-hand side (pivots, and the border entries of this
+// workgroup's rows) from r and the children's updates, by a list of update
+// entries for each front entry; then update = rhs_q - W rhs_p.
+__global__ void __launch_bounds__(ND_NT) k_nd_up(const NdTask *__restrict__ tasks, const int *__restrict__ piv,
+                                                 const int *__restrict__ sptr, const int *__restrict__ src,
+                                                 const double *__restrict__ fac, const double *__restrict__ r,
+                                                 double *__restrict__ y, double *upd) {
     extern __shared__ double nd_v[];
-    const int4 t = tasks[blockIdx.x];
-    const NdDev N = nodes[t.x];
-    for (int i = threadIdx.x; i < N.p + N.q; i += ND_NT) nd_v[i] = i < N.p ? r[piv[N.po + i]] : 0.0;
-    for (int c = N.kid0; c < N.kid1; c++) {
-        const NdDev C = nodes[kids[c]];
-        __syncthreads();
-        for (int j = threadIdx.x; j < C.q; j += ND_NT) nd_v[cmap[C.bo + j]] += upd[C.bo + j];
-    }
-    __syncthreads();
-    if (t.y == 0)
-        for (int i = threadIdx.x; i < N.p; i += ND_NT) y[N.po + i] = nd_v[i];
-    auto put = [&](int row, double s) { upd[N.bo + row] = nd_v[N.p + row] - s; };
-    if (N.p > 256)
-        nd_rows<64>(fac + N.w, N.p, t.y, t.z, nd_v, put);
-    else
-        nd_rows<16>(fac + N.w, N.p, t.y, t.z, nd_v, put);
+    const NdTask T = tasks[blockIdx.x];
+    auto gather = [&] {
+        const int n = T.p + T.row1 - T.row0;
+        for (int i = threadIdx.x; i < n; i += ND_NT) {
+            const int f = T.fo + (i < T.p ? i : i + T.row0);
+            double x = i < T.p ? r[piv[T.po + i]] : 0.0;
+            for (int e = sptr[f]; e < sptr[f + 1]; e++) x += upd[src[e]];
+            nd_v[i] = x;
+            if (i < T.p && T.row0 == 0) y[T.po + i] = x;
+        }
+    };
+    nd_dispatch(T, fac, T.p, nd_v, gather, [&](int row, double s) { upd[T.bo + row] = nd_v[T.p + row - T.row0] - s; });
 }
 
 // Down: x_p = [inv(F11) | -U] [rhs_p ; x_q]; z holds the correction by
 // matrix row for the nodes below, x takes it.
-__global__ void __launch_bounds__(ND_NT) k_nd_down(const int4 *__restrict__ tasks, const NdDev *__restrict__ nodes,
-                                                   const int *__restrict__ piv, const int *__restrict__ border,
-                                                   const double *__restrict__ fac, const double *__restrict__ y,
-                                                   double *z, double *__restrict__ x) {
+__global__ void __launch_bounds__(ND_NT) k_nd_down(const NdTask *__restrict__ tasks, const int *__restrict__ piv,
+                                                   const int *__restrict__ border, const double *__restrict__ fac,
+                                                   const double *__restrict__ y, double *z, double *__restrict__ x) {
     extern __shared__ double nd_v[];
-    const int4 t = tasks[blockIdx.x];
-    const NdDev N = nodes[t.x];
-    const int m = N.p + N.q;
-    for (int i = threadIdx.x; i < m; i += ND_NT) nd_v[i] = i < N.p ? y[N.po + i] : z[border[N.bo + i - N.p]];
-    __syncthreads();
-    auto put = [&](int row, double s) {
-        const int g = piv[N.po + row];
+    const NdTask T = tasks[blockIdx.x];
+    const int m = T.p + T.q;
+    auto gather = [&] {
+        constexpr int U = 8;
+        for (int i0 = threadIdx.x; i0 < m; i0 += U * ND_NT) {
+            int g[U];
+            double x[U];
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                const int i = i0 + q * ND_NT;
+                g[q] = i >= T.p && i < m ? border[T.bo + i - T.p] : -1;
+            }
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                const int i = i0 + q * ND_NT;
+                x[q] = g[q] >= 0 ? z[g[q]] : i < T.p ? y[T.po + i] : 0.0;
+            }
+#pragma unroll
+            for (int q = 0; q < U; q++)
+                if (i0 + q * ND_NT < m) nd_v[i0 + q * ND_NT] = x[q];
+        }
+    };
+    nd_dispatch(T, fac, m, nd_v, gather, [&](int row, double s) {
+        const int g = piv[T.po + row];
         z[g] = s;
         x[g] += s;
-    };
-    if (m > 256)
-        nd_rows<64>(fac + N.g, m, t.y, t.z, nd_v, put);
-    else
-        nd_rows<16>(fac + N.g, m, t.y, t.z, nd_v, put);
+    });
 }
 
 class NdSolver {
@@ -520,61 +556,81 @@ class NdSolver {
         entries = T.entries;
         if (T.flops > max_flops || T.entries > max_entries) return false;
         for (const NdNode &N : T.nodes)
-            if ((int)(N.piv.size() + N.border.size()) > ND_LDS) return false;
+            if ((int)(N.piv.size() + N.border.size()) > ND_LDS - ND_NT / 8) return false;
         if (!T.numeric(rp, ci, v)) return false;
         const int nn = (int)T.nodes.size();
-        std::vector<NdDev> dv(nn);
-        std::vector<int> kids, piv, border, cmap;
+        std::vector<int> piv, border, sptr(1, 0), src, bo(nn, 0);
         std::vector<double> fac;
         fac.reserve((size_t)T.entries);
-        std::vector<std::vector<int4>> up(T.height), down(T.height);
+        std::vector<std::vector<NdTask>> up(T.height), down(T.height);
         height_ = T.height;
-        lds_.assign(height_, 0);
+        ulds_.assign(height_, 0);
+        dlds_.assign(height_, 0);
+        std::vector<std::vector<int>> from;
         for (int q = 0; q < nn; q++) {
             NdNode &N = T.nodes[q];
-            NdDev &d = dv[q];
-            d.p = (int)N.piv.size();
-            d.q = (int)N.border.size();
-            d.po = (int)piv.size();
-            d.bo = (int)border.size();
-            d.kid0 = (int)kids.size();
-            kids.insert(kids.end(), N.child.begin(), N.child.end());
-            d.kid1 = (int)kids.size();
+            NdTask t;
+            t.p = (int)N.piv.size();
+            t.q = (int)N.border.size();
+            t.po = (int)piv.size();
+            t.bo = bo[q] = (int)border.size();
+            t.fo = (int)sptr.size() - 1;
+            const int m = t.p + t.q;
+            // the children's update entries of each front entry, in the
+            // children's order
+            from.assign(m, {});
+            for (int c : N.child)
+                for (size_t k = 0; k < T.nodes[c].cmap.size(); k++) from[T.nodes[c].cmap[k]].push_back(bo[c] + (int)k);
+            for (auto &f : from) {
+                src.insert(src.end(), f.begin(), f.end());
+                sptr.push_back((int)src.size());
+            }
             piv.insert(piv.end(), N.piv.begin(), N.piv.end());
             border.insert(border.end(), N.border.begin(), N.border.end());
-            cmap.insert(cmap.end(), N.cmap.begin(), N.cmap.end());
-            cmap.resize(border.size(), 0);  // a root's (empty) border has no map
-            d.w = (long)fac.size();
+            auto cut = [&](int rows, int len, long at, std::vector<NdTask> &out) {
+                t.at = at;
+                t.gl = nd_lanes(len);
+                const int step = ND_NT / t.gl;
+                for (t.row0 = 0; t.row0 < std::max(rows, 1); t.row0 += step) {
+                    t.row1 = std::min(rows, t.row0 + step);
+                    out.push_back(t);
+                }
+            };
+            if (t.q > 0) {
+                cut(t.q, t.p, (long)fac.size(), up[N.height]);
+            } else {  // a root only gathers: 256 pivots per workgroup
+                NdTask c = t;
+                c.row0 = c.row1 = 0;
+                c.at = 0;
+                c.gl = 64;
+                for (int k = 0; k < t.p; k += ND_NT) {
+                    c.po = t.po + k;
+                    c.fo = t.fo + k;
+                    c.p = std::min(ND_NT, t.p - k);
+                    up[N.height].push_back(c);
+                }
+            }
+            ulds_[N.height] = std::max(ulds_[N.height], t.p + ND_NT / 8);
             fac.insert(fac.end(), N.W.begin(), N.W.end());
-            d.g = (long)fac.size();
+            cut(t.p, m, (long)fac.size(), down[N.height]);
+            dlds_[N.height] = std::max(dlds_[N.height], m);
             fac.insert(fac.end(), N.G.begin(), N.G.end());
             std::vector<double>().swap(N.W);
             std::vector<double>().swap(N.G);
-            const int m = d.p + d.q;
-            lds_[N.height] = std::max(lds_[N.height], m);
-            // about 8192 factor entries per workgroup, 16 to 64 rows
-            auto cut = [&](int rows, int len, std::vector<int4> &out) {
-                const int step = std::max(16, std::min(64, 8192 / std::max(len, 1) / 16 * 16));
-                for (int r = 0; r < std::max(rows, 1); r += step)
-                    out.push_back(make_int4(q, r, std::min(rows, r + step), 0));
-            };
-            cut(d.q, d.p, up[N.height]);
-            cut(d.p, m, down[N.height]);
         }
         up_.assign(height_ + 1, 0);
         down_.assign(height_ + 1, 0);
-        std::vector<int4> ut, dt;
+        std::vector<NdTask> ut, dt;
         for (int h = 0; h < height_; h++) {
             ut.insert(ut.end(), up[h].begin(), up[h].end());
             dt.insert(dt.end(), down[h].begin(), down[h].end());
             up_[h + 1] = (int)ut.size();
             down_[h + 1] = (int)dt.size();
         }
-        put(nodes_, dv, st);
-        put(kids_, kids, st);
         put(piv_, piv, st);
         put(border_, border, st);
-        put(cmap_, cmap, st);
+        put(sptr_, sptr, st);
+        put(src_, src, st);
         put(fac_, fac, st);
         put(ut_, ut, st);
         put(dt_, dt, st);
@@ -589,19 +645,18 @@ class NdSolver {
     // x += A^-1 r
     void correct(const double *r, double *x, hipStream_t st) {
         for (int h = 0; h < height_; h++)
-            k_nd_up<<<up_[h + 1] - up_[h], ND_NT, lds_[h] * sizeof(double), st>>>(ut_.p + up_[h], nodes_.p, kids_.p, piv_.p,
-                                                                                cmap_.p, fac_.p, r, y_.p, updv_.p);
+            k_nd_up<<<up_[h + 1] - up_[h], ND_NT, ulds_[h] * sizeof(double), st>>>(ut_.p + up_[h], piv_.p, sptr_.p, src_.p,
+                                                                                 fac_.p, r, y_.p, updv_.p);
         for (int h = height_ - 1; h >= 0; h--)
-            k_nd_down<<<down_[h + 1] - down_[h], ND_NT, lds_[h] * sizeof(double), st>>>(
-                dt_.p + down_[h], nodes_.p, piv_.p, border_.p, fac_.p, y_.p, z_.p, x);
+            k_nd_down<<<down_[h + 1] - down_[h], ND_NT, dlds_[h] * sizeof(double), st>>>(
+                dt_.p + down_[h], piv_.p, border_.p, fac_.p, y_.p, z_.p, x);
     }
 
   private:
     int height_ = 0;
-    std::vector<int> up_, down_, lds_;
-    KBuf<NdDev> nodes_;
-    KBuf<int> kids_, piv_, border_, cmap_;
-    KBuf<int4> ut_, dt_;
+    std::vector<int> up_, down_, ulds_, dlds_;
+    KBuf<int> piv_, border_, sptr_, src_;
+    KBuf<NdTask> ut_, dt_;
     KBuf<double> fac_, y_, updv_, z_;
 
     template <typename T>
