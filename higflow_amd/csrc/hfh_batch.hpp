@@ -308,10 +308,9 @@ int Flow<D>::member_field(int m, int field, int comp, double *buf, bool set) {
     int off = remap(m, f.field_offset(field, comp));
     if (set) extrap_hist_ = 0;
     if (set)
-        HFH_CHECK(hipMemcpyAsync(X_.p + off, buf, sizeof(double) * n, hipMemcpyHostToDevice, st_));
+        stage_.write(X_.p + off, buf, n, st_);
     else
-        HFH_CHECK(hipMemcpyAsync(buf, X_.p + off, sizeof(double) * n, hipMemcpyDeviceToHost, st_));
-    HFH_CHECK(hipStreamSynchronize(st_));
+        stage_.read(buf, X_.p + off, n, st_);
     return n;
 }
 

@@ -365,6 +365,7 @@ class Flow : public FlowBase {
     // sizes the step is latency-bound, and the FP32 right-hand sides cost
     // solver iterations.
     bool k32_ = false;
+    HostStage stage_;  // field exchange
     DevBuf<int> dMomSlots_[D], dVeSlots_;
     DevBuf<unsigned> dMomFlags_[D], dVeFlags_;
     DevBuf<double> dMomDelta_[D], dVeDelta_;

@@ -1282,8 +1282,7 @@ int Flow<D>::get_field(int field, int comp, double *out) {
     int n = field_size(field, comp);
     if (n < 0 || host_only_ || !mem_.empty()) return -1;
     const double *src = field == 9 ? poly_stress(comp) : X_.p + field_offset(field, comp);
-    HFH_CHECK(hipMemcpyAsync(out, src, sizeof(double) * n, hipMemcpyDeviceToHost, st_));
-    HFH_CHECK(hipStreamSynchronize(st_));
+    stage_.read(out, src, n, st_);
     return n;
 }
 
@@ -1314,8 +1313,7 @@ int Flow<D>::set_field(int field, int comp, const double *in) {
     if (field == 6 && comp / D > comp % D) return n;  // symmetric storage keeps the upper triangle
     int off = field_offset(field, comp);
     extrap_hist_ = 0;
-    HFH_CHECK(hipMemcpyAsync(X_.p + off, in, sizeof(double) * n, hipMemcpyHostToDevice, st_));
-    HFH_CHECK(hipStreamSynchronize(st_));
+    stage_.write(X_.p + off, in, n, st_);
     return n;
 }
 
