@@ -404,6 +404,169 @@ __global__ void __launch_bounds__(FDM_NT) k_fdm(const int4 *__restrict__ tiles, 
     }
 }
 
+// ------------------------------------------------------------ small systems
+// The whole pass (residual, the 2 D products, x += z, new residual, norms) of
+// a system of up to 2048 rows in one workgroup, in LDS: seven launches and the
+// gaps between them are all that a system of this size costs otherwise.  One
+// CU catches up with them near 48^2 and 14^3 rows; a time step of an explicit
+// cavity takes, with launches and in one workgroup, 80 and 66 us at 32^2,
+// 81 and 77 at 44^2, 81 and 95 at 64^2; in 3D 95 and 75 us at 8^3, 99 and 88
+// at 12^3, 117 and 131 at 16^3.
+struct FdmSmall {
+    int off, n[3];
+    int ld;        // row stride in LDS: odd, so 16 rows fall on 16 bank pairs
+    int l[3];      // eigenvalue tables
+    long v[3];     // V of each dimension; V^T follows it
+};
+constexpr int FDM_SMALL = 2048;
+constexpr int FDM_SNT = 1024;
+
+// one product along dimension DIM over the LDS array src, 16 x 16 tiles
+// round robin over the waves; out(m, n, tile's z plane, LDS index, value)
+template <int DIM, typename Out>
+__device__ inline void fdm_small_stage(const FdmSmall &J, const double *__restrict__ mat, const double *src, Out &&out) {
+    const int nx = J.n[0], ny = J.n[1], nz = J.n[2], ld = J.ld, lz = ld * ny;
+    const int M = DIM == 0 ? ny * nz : DIM == 1 ? ny : nz, N = DIM == 2 ? nx * ny : nx, K = J.n[DIM];
+    const int tm = (M + 15) / 16, tn = (N + 15) / 16, planes = DIM == 1 ? nz : 1;
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    for (int t = threadIdx.x >> 6; t < tm * tn * planes; t += FDM_SNT / 64) {
+        const int z = t / (tm * tn), m0 = (t / tn) % tm * 16, n0 = t % tn * 16;
+        const int m = min(m0 + li, M - 1), n = min(n0 + li, N - 1);
+        const int nat = DIM == 2 ? n / nx * ld + n % nx : n;
+        fdm_d4 c = {0, 0, 0, 0};
+        constexpr int U = 4;
+        for (int k0 = 0; k0 < K; k0 += 4 * U) {
+            double a[U], b[U];
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                const int k = k0 + 4 * q + lk, kc = min(k, K - 1);
+                a[q] = DIM == 0 ? src[m * ld + kc] : mat[kc * K + m];
+                b[q] = DIM == 0 ? mat[kc * K + n] : DIM == 1 ? src[z * lz + kc * ld + n] : src[kc * lz + nat];
+                if (k >= K) a[q] = b[q] = 0.0;
+            }
+#pragma unroll
+            for (int q = 0; q < U; q++) {
+                if (k0 + 4 * q >= K) break;  // the same for the whole wave
+                c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b[q], c, 0, 0, 0);
+            }
+        }
+        if (n0 + li >= N) continue;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int row = m0 + 4 * q + lk;
+            if (row < M) out(row, n0 + li, z, DIM == 0 ? row * ld + n : DIM == 1 ? z * lz + row * ld + n : row * lz + nat, c[q]);
+        }
+    }
+    __syncthreads();
+}
+
+// sums of three values over the workgroup, on every thread
+__device__ inline void fdm_small_sums(double (&v)[3], double (*sh)[FDM_SNT / 64]) {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+        if ((threadIdx.x & 63) == 0) sh[k][threadIdx.x >> 6] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        v[k] = 0;
+        for (int q = 0; q < FDM_SNT / 64; q++) v[k] += sh[k][q];
+    }
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(FDM_SNT) k_fdm_small(const FdmSmall *__restrict__ jobs, const FdmPin *__restrict__ pins,
+                                                       int nd, KRows<double> A, const double *__restrict__ mats,
+                                                       const double *__restrict__ lam, const double *__restrict__ g,
+                                                       const double *__restrict__ dinv, const double *__restrict__ b,
+                                                       double *__restrict__ x, double *norms) {
+    extern __shared__ double fdm_lds[];
+    __shared__ double sh[3][FDM_SNT / 64];
+    __shared__ double s_rp;
+    const FdmSmall J = jobs[blockIdx.x];
+    const FdmPin P = pins[blockIdx.x];
+    const int nx = J.n[0], ny = J.n[1], nz = J.n[2], N = nx * ny * nz, ld = J.ld, size = ld * ny * nz;
+    double *u = fdm_lds, *w = fdm_lds + size;
+    // b - A x of local row i of the stored matrix; at(j) is x of local row j
+    auto residual = [&](int i, auto &&at) {
+        const int gi = J.off + i, t = A.code ? A.code[gi] : -1;
+        double s = 0;
+        if (A.dw && t >= 0) {
+            const int *db = A.dblk + (size_t)(gi / KNT) * (KD_MAX + 1);
+            const unsigned msk = A.dmask[t];
+            for (int e = 0; e < KD_MAX; e++)
+                if ((msk >> e) & 1u) s += A.dw[(size_t)t * KD_MAX + e] * at(i + db[e]);
+        } else {
+            for (int k = A.rp[gi]; k < A.rp[gi + 1]; k++) s += A.val[k] * at(A.ci[k] - J.off);
+        }
+        return b[gi] - s;
+    };
+    double v[3] = {0, 0, 0};  // sum r
+    for (int i = threadIdx.x; i < N; i += FDM_SNT) {
+        const double r = residual(i, [&](int j) { return x[J.off + j]; });
+        u[i / nx * ld + i % nx] = r;
+        v[0] += r;
+        if (i == P.pin) s_rp = r;
+    }
+    fdm_small_sums(v, sh);
+    const double mu = -v[0], rp = P.pin >= 0 ? s_rp : 0.0;
+    auto to = [](double *d) { return [d](int, int, int, int at, double c) { d[at] = c; }; };
+    // V^T r along every dimension, over the eigenvalue sums, and back
+    auto scaled = [&](double *d) {
+        return [&, d](int m, int n, int z, int at, double c) {
+            // 2D: (ky, kx) = (m, n); 3D: kz = m, n = (ky, kx)
+            const double l = nd == 3 ? (lam[J.l[0] + n % nx] + lam[J.l[1] + n / nx]) + lam[J.l[2] + m]
+                                     : lam[J.l[0] + n] + lam[J.l[1] + m];
+            d[at] = P.pin >= 0 && m == 0 && n == 0 ? 0.0 : c / l;
+        };
+    };
+    const double *V[3], *Z[3];
+    for (int d = 0; d < 3; d++) {
+        V[d] = mats + J.v[d];
+        Z[d] = V[d] + (long)J.n[d] * J.n[d];
+    }
+    fdm_small_stage<0>(J, V[0], u, to(w));
+    if (nd == 3) {
+        fdm_small_stage<1>(J, V[1], w, to(u));
+        fdm_small_stage<2>(J, V[2], u, scaled(w));
+        fdm_small_stage<2>(J, Z[2], w, to(u));
+        fdm_small_stage<1>(J, Z[1], u, to(w));
+    } else {
+        fdm_small_stage<1>(J, V[1], w, scaled(u));
+        fdm_small_stage<1>(J, Z[1], u, to(w));
+    }
+    double c = 0, zp = 0;
+    if (P.pin >= 0) {  // as k_fdm
+        double t[3] = {0, 0, 0};
+        for (int k = threadIdx.x; k < nx; k += FDM_SNT) t[0] += w[P.rowp * ld + k] * V[0][(size_t)P.colp * nx + k];
+        fdm_small_sums(t, sh);
+        const double own = rp * dinv[J.off + P.pin];
+        zp = P.mode == FDM_PIN_SHIFT ? -mu / P.shift : P.mode == FDM_PIN_ROW ? own : 0.0;
+        c = zp - t[0] - mu * g[J.off + P.pin];
+        if (P.mode == FDM_PIN_ELIM) zp = own;
+    }
+    // the new x stays in LDS (u, without the padding) for its residual
+    fdm_small_stage<0>(J, Z[0], w, [&](int m, int n, int, int, double z) {
+        const int i = m * nx + n, gi = J.off + i;
+        if (P.pin >= 0) z = i == P.pin ? zp : z + (mu * g[gi] + c);
+        const double xn = x[gi] + z;
+        x[gi] = xn;
+        u[i] = xn;
+    });
+    double q[3] = {0, 0, 0};
+    for (int i = threadIdx.x; i < N; i += FDM_SNT) {
+        const double r = residual(i, [&](int j) { return u[j]; }), bi = b[J.off + i];
+        q[0] += r * r;
+        q[1] += bi * bi;
+    }
+    fdm_small_sums(q, sh);
+    if (threadIdx.x == 0) {
+        norms[2 * blockIdx.x] = q[0];
+        norms[2 * blockIdx.x + 1] = q[1];
+    }
+}
+
 // r.r and b.b of each segment from the 256-row partials, written to pinned
 // host memory (one workgroup per segment)
 __global__ void __launch_bounds__(256) k_seg_norms(const int *__restrict__ w0, const double *__restrict__ prr,
@@ -438,6 +601,7 @@ class FdmSolver {
   public:
     bool ready = false;
     int n = 0, nd = 0, nsys = 0;
+    bool small = false;  // every system fits one workgroup (pass_small)
 
     // segments as DeviceSystem::set_matrix takes them; false (no plan) when
     // a segment has no Kronecker form, or no coupling reaches min_coupling
@@ -480,6 +644,9 @@ class FdmSolver {
         };
         std::vector<FdmJob> jobs;
         std::vector<FdmPin> pins(nsys);
+        std::vector<FdmSmall> sm(nsys);
+        small = true;
+        small_lds_ = 0;
         std::vector<std::vector<int4>> tl(2 * nd);
         bool pinned = false;
         for (int q = 0; q < nsys; q++) {
@@ -494,6 +661,16 @@ class FdmSolver {
                 for (double c : e.second) lam.push_back(s.a / nd + s.b[d] * c);
             }
             const int nx = s.n[0], ny = s.n[1], nz = s.n[2], nxy = nx * ny;
+            FdmSmall &j = sm[q];
+            j.off = s.off;
+            j.ld = nx | 1;
+            for (int d = 0; d < 3; d++) {
+                j.n[d] = s.n[d];
+                j.l[d] = L[d];
+                j.v[d] = V[d];
+            }
+            small = small && nxy * nz <= FDM_SMALL;
+            small_lds_ = std::max(small_lds_, 2 * (size_t)j.ld * ny * nz * sizeof(double));
             auto add = [&](int stage, int M, int N, int K, int lda, int ldb, int ldc, int batch, int bstride, long moff) {
                 FdmJob j;
                 j.M = M, j.N = N, j.K = K, j.lda = lda, j.ldb = ldb, j.ldc = ldc;
@@ -537,6 +714,12 @@ class FdmSolver {
             ntiles_[q] = (int)tl[q].size();
             put(tiles_[q], tl[q], st);
         }
+        if (small) {
+            put(small_, sm, st);
+            if (hipFuncSetAttribute(reinterpret_cast<const void *>(k_fdm_small), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)small_lds_) != hipSuccess)
+                small = false;
+        }
         put(jobs_, jobs, st);
         put(pins_, pins, st);
         put(mats_, pool, st);
@@ -564,7 +747,16 @@ class FdmSolver {
         stages(r, x, psum, dinv, st, true);
     }
 
+    // x += M (b - A x) and the norms of the new residual and of b, with one
+    // workgroup per system
+    void pass_small(const KRows<double> &A, const double *dinv, const double *b, double *x, double *norms,
+                    hipStream_t st) {
+        k_fdm_small<<<nsys, FDM_SNT, small_lds_, st>>>(small_.p, pins_.p, nd, A, mats_.p, lam_.p, g_.p, dinv, b, x, norms);
+    }
+
   private:
+    KBuf<FdmSmall> small_;
+    size_t small_lds_ = 0;
     KBuf<int4> tiles_[6];
     int ntiles_[6] = {0, 0, 0, 0, 0, 0};
     KBuf<FdmJob> jobs_;

@@ -840,18 +840,24 @@ class DeviceSystem {
     // passes the stopping test or stops falling.  False when the corrections
     // do not converge (the caller goes on with the Krylov solver from x).
     bool direct_solve(const double *b, double *x, double rtol, double atol, hipStream_t st, SolveStats &S) {
-        const double *h = reinterpret_cast<const double *>(hpin_ + off_fd_);
+        double *norms = reinterpret_cast<double *>(hpin_ + off_fd_);
+        const double *h = norms;
         std::vector<SolveStats> gs(nseg);
         double best = -1.0;
-        true_residual(x, b, st);
+        const bool small = fdm.ready && fdm.small;
+        if (!small) true_residual(x, b, st);
         for (int pass = 1; pass <= 4; pass++) {
             if (pass > 1) HFH_CHECK(hipMemcpyAsync(xbak.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
-            if (fdm.ready)
-                fdm.correct(r.p, x, part3.p, dinv.p, st);
-            else
-                nd.correct(r.p, x, st);
-            true_residual(x, b, st);
-            k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part2.p, reinterpret_cast<double *>(hpin_ + off_fd_));
+            if (small) {
+                fdm.pass_small(k64.Av, dinv.p, b, x, norms, st);
+            } else {
+                if (fdm.ready)
+                    fdm.correct(r.p, x, part3.p, dinv.p, st);
+                else
+                    nd.correct(r.p, x, st);
+                true_residual(x, b, st);
+                k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part2.p, norms);
+            }
             HFH_CHECK(hipStreamSynchronize(st));
             bool all_conv = true;
             double worst = 0;

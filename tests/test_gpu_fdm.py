@@ -70,13 +70,15 @@ def test_end_rows(ends):
 
 
 @pytest.mark.parametrize("sizes", [(3, 3), (4, 5), (15, 17), (31, 33), (32, 32), (33, 3), (3, 64), (65, 20),
-                                   (3, 3, 3), (5, 4, 6), (11, 33, 3), (33, 3, 9)])
+                                   (3, 3, 3), (5, 4, 6), (11, 33, 3), (33, 3, 9),
+                                   # one workgroup up to 2048 rows, tiles of many above
+                                   (64, 32), (45, 46), (33, 65), (8, 16, 16), (12, 12, 15)])
 def test_box_sizes(sizes):
     b = np.random.default_rng(2).normal(size=int(np.prod(sizes)))
     _check(_box(sizes, ["NH", "DD", "HN"][:len(sizes)], shift=0.1), b)
 
 
-@pytest.mark.parametrize("sizes", [(8, 6), (33, 12), (5, 6, 7)])
+@pytest.mark.parametrize("sizes", [(8, 6), (33, 12), (5, 6, 7), (49, 43), (13, 12, 14)])
 @pytest.mark.parametrize("mode", ["eliminated", "imposed", "shifted"])
 @pytest.mark.parametrize("where", ["first", "inside", "last"])
 def test_special_unknown(sizes, mode, where):
