@@ -845,6 +845,7 @@ int Flow<D>::step(bool ve) {
     if (par_.tempdiscrtype != EXPLICIT_EULER && par_.tempdiscrtype != SEMI_IMPLICIT_EULER) return -3;
     const bool semi = par_.tempdiscrtype == SEMI_IMPLICIT_EULER;
     if (ve != (par_.flowtype == VISCOELASTIC)) return -4;
+    psys_.early = hsysB_.early = nullptr;
     if (!ve) {
         boundary_refresh();
         source_refresh();
@@ -900,8 +901,10 @@ int Flow<D>::step(bool ve) {
     run_group(dMom_, 1.0, X, ST_INTERP);
     tend(ST_INTERP);
     tbegin(ST_MOMENTUM);
+    MomSet<D> ms;
+    int nfmax = 0;
     for (int d = 0; d < D; d++) {
-        MomParams mp;
+        MomParams &mp = ms.p[d];
         mp.nf = Nf_[d];
         mp.ns = momNs_;
         mp.u_off = oU_[d];
@@ -916,13 +919,16 @@ int Flow<D>::step(bool ve) {
         mp.bout = semi ? (hbatched_ ? hbB_.p + hoff_[d] : hb_[d].p) : nullptr;
         mp.bcst = semi ? hcst_[d].p : nullptr;
         mp.re = momRe_[d].empty() ? nullptr : dMomRe_[d].p;
-        if (mp.nf > 0 && k32_)
-            k_momentum<D, float><<<nblocks(mp.nf), BLOCK, 0, st_>>>(mp, dMomSlots_[d].p, dMomFlags_[d].p,
-                                                                    dMomDelta_[d].p, X);
-        else if (mp.nf > 0)
-            k_momentum<D><<<nblocks(mp.nf), BLOCK, 0, st_>>>(mp, dMomSlots_[d].p, dMomFlags_[d].p, dMomDelta_[d].p,
-                                                             X);
+        ms.slots[d] = dMomSlots_[d].p;
+        ms.flags[d] = dMomFlags_[d].p;
+        ms.delta[d] = dMomDelta_[d].p;
+        nfmax = std::max(nfmax, mp.nf);
     }
+    if (nfmax > 0 && k32_)
+        k_momentum<D, float><<<dim3(nblocks(nfmax), D), BLOCK, 0, st_>>>(ms, X);
+    else if (nfmax > 0)
+        k_momentum<D><<<dim3(nblocks(nfmax), D), BLOCK, 0, st_>>>(ms, X);
+    bool div_done = false;
     if (semi && hbatched_) {
         // the D Helmholtz systems in the same launches, warm-started from
         // the last u*; one stopping test per component
@@ -944,11 +950,20 @@ int Flow<D>::step(bool ve) {
         // one launch for the D components: initial guesses, then (after the
         // solve) the copy back into u*
         if (nmax > 0) k_extrap_set<<<dim3(nblocks(nmax), D), BLOCK, 0, st_>>>(es, std::min(extrap_, extrap_hist_));
+        // a direct solve enqueues the copy into u* and the divergence rows
+        // behind its first pass, before it waits for that pass's norms
+        auto after = [&] {
+            if (nmax > 0) k_copy_set<<<dim3(nblocks(nmax), D), BLOCK, 0, st_>>>(cs);
+            run_group(dDiv_, 1.0, bvec_.p, ST_DIV);
+        };
+        if (!timing_on_) hsysB_.early = after;
         if (par_.precision == 1)
             hsysB_.fused_mixed(spd, hbB_.p, hxB_.p, par_.rtol, par_.atol, par_.inner_rtol, par_.maxit, st_);
         else
             hsysB_.fused64(spd, hbB_.p, hxB_.p, par_.rtol, par_.atol, par_.maxit, st_);
-        if (nmax > 0) k_copy_set<<<dim3(nblocks(nmax), D), BLOCK, 0, st_>>>(cs);
+        hsysB_.early = nullptr;
+        div_done = hsysB_.early_done;
+        if (!div_done && nmax > 0) k_copy_set<<<dim3(nblocks(nmax), D), BLOCK, 0, st_>>>(cs);
         for (int d = 0; d < D; d++)
             if ((int)hsysB_.seg_stats.size() == D) hstats_[d] = hsysB_.seg_stats[d];
     } else if (semi) {  // one Helmholtz solve per component, warm-started from the last u*
@@ -970,12 +985,16 @@ int Flow<D>::step(bool ve) {
     }
     tend(ST_MOMENTUM);
     tbegin(ST_DIV);
-    run_group(dDiv_, 1.0, bvec_.p, ST_DIV);
+    if (!div_done) run_group(dDiv_, 1.0, bvec_.p, ST_DIV);
     tend(ST_DIV);
     tbegin(ST_SOLVE);
     double *x = X + (par_.projtype == INCREMENTAL ? oDP_ : oP_);
     if (extrap_)
         k_extrap<double><<<nblocks(Nc_), BLOCK, 0, st_>>>(Nc_, x, pPrev_.p, pPrev2_.p, x, std::min(extrap_, extrap_hist_));
+    // likewise the projection rows (they write u from u* and the increment,
+    // so running them again after a second pass is harmless)
+    if (!timing_on_) psys_.early = [&] { run_group(dGrad_, -par_.dt, X, ST_PROJECT); };
+    psys_.early_done = false;
     if (psys_.fused && par_.precision == 1) {
         stats_ = psys_.fused_mixed(symmetric_, bvec_.p, x, par_.rtol, par_.atol, par_.inner_rtol, par_.maxit, st_);
     } else if (psys_.fused) {
@@ -987,9 +1006,10 @@ int Flow<D>::step(bool ve) {
     } else {
         stats_ = psys_.bicgstab(bvec_.p, x, par_.rtol, par_.atol, par_.maxit, st_);
     }
+    psys_.early = nullptr;
     tend(ST_SOLVE);
     tbegin(ST_PROJECT);
-    run_group(dGrad_, -par_.dt, X, ST_PROJECT);
+    if (!psys_.early_done) run_group(dGrad_, -par_.dt, X, ST_PROJECT);
     if (par_.projtype == INCREMENTAL) k_axpy_field<double><<<nblocks(Nc_), BLOCK, 0, st_>>>(Nc_, X, oP_, oDP_);
     tend(ST_PROJECT);
     par_.t += par_.dt;
@@ -1029,6 +1049,7 @@ int Flow<D>::probe(int which, int reps, double *avg_ms, long *bytes) {
     double *X = X_.p;
     long by = 0;
     int n = Nc_;
+    MomSet<D> pm{};
     MomParams mp;
     mp.nf = Nf_[0];
     mp.ns = momNs_;
@@ -1150,8 +1171,11 @@ int Flow<D>::probe(int which, int reps, double *avg_ms, long *bytes) {
             return 0;
         }
         case 1:
-            k_momentum<D><<<nblocks(mp.nf), BLOCK, 0, st_>>>(mp, dMomSlots_[0].p, dMomFlags_[0].p,
-                                                             dMomDelta_[0].p, X);
+            pm.p[0] = mp;
+            pm.slots[0] = dMomSlots_[0].p;
+            pm.flags[0] = dMomFlags_[0].p;
+            pm.delta[0] = dMomDelta_[0].p;
+            k_momentum<D><<<nblocks(mp.nf), BLOCK, 0, st_>>>(pm, X);
             by = (long)mp.nf * ((long)momNs_ * (4 + 8) + 4 + D * 8 + 8 + 8);
             break;
         case 2:

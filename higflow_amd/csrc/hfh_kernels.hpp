@@ -297,10 +297,20 @@ struct MomParams {
 //   velocities, then D tensor divergences (viscoelastic).
 // flags: bits 0-1 final convective type, bit 2+d2 infacet_rr, bit 2+D+d2
 // infacet_ll (hig-flow-discret.c:131-251).
+// One launch for all components (blockIdx.y).
+template <int D>
+struct MomSet {
+    MomParams p[D];
+    const int *slots[D];
+    const unsigned *flags[D];
+    const double *delta[D];
+};
 template <int D, typename C = double>
-__global__ void __launch_bounds__(BLOCK) k_momentum(MomParams P, const int *__restrict__ slots,
-                                                    const unsigned *__restrict__ flags,
-                                                    const double *__restrict__ fdelta, double *X) {
+__global__ void __launch_bounds__(BLOCK) k_momentum(MomSet<D> M, double *X) {
+    const MomParams &P = M.p[blockIdx.y];
+    const int *__restrict__ slots = M.slots[blockIdx.y];
+    const unsigned *__restrict__ flags = M.flags[blockIdx.y];
+    const double *__restrict__ fdelta = M.delta[blockIdx.y];
     int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= P.nf) return;
     const int nf = P.nf;

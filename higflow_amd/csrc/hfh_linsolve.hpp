@@ -19,6 +19,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -577,6 +578,11 @@ class DeviceSystem {
     // the direct solve wants a coupling of at least this share of the diagonal
     double fdm_min_coupling = 0;
     bool direct() const { return fdm.ready || nd.ready; }
+    // work that follows the solve on the stream: a direct solve enqueues it
+    // behind its first pass, before the wait; early_done tells whether that
+    // was the last word on x (else the caller runs it after the solve)
+    std::function<void()> early;
+    bool early_done = false;
     bool fused = true;
     int max_restarts = 1;      // fused64: restarts on the true residual
     double t_mixed_ = -1, t_fp64_ = -1;  // mixed form: seconds per solve of each form
@@ -858,6 +864,8 @@ class DeviceSystem {
                 true_residual(x, b, st);
                 k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part2.p, norms);
             }
+            if (pass == 1 && early) early();
+            early_done = pass == 1 && early;
             HFH_CHECK(hipStreamSynchronize(st));
             bool all_conv = true;
             double worst = 0;
@@ -911,9 +919,11 @@ class DeviceSystem {
     // passes, the true residual b - A x is checked and the iteration
     // restarted from x (at most twice) while it misses the tolerance.
     SolveStats fused64(bool spd, const double *b, double *x, double rtol, double atol, int maxit, hipStream_t st) {
+        early_done = false;
         if (direct() && maxit > 0) {
             SolveStats F;
             if (direct_solve(b, x, rtol, atol, st, F)) return F;
+            early_done = false;
             fdm.ready = nd.ready = false;
         }
         ensure_amg(st);
@@ -1074,6 +1084,7 @@ class DeviceSystem {
     // all segments together, each against its own tolerance.
     SolveStats fused_mixed(bool spd, const double *b, double *x, double rtol, double atol, double inner_rtol,
                            int maxit, hipStream_t st) {
+        early_done = false;
         if (direct() && maxit > 0) {
             SolveStats F;
             if (direct_solve(b, x, rtol, atol, st, F)) {
@@ -1081,6 +1092,7 @@ class DeviceSystem {
                 for (auto &g : seg_stats) g.fallback = 2;
                 return F;
             }
+            early_done = false;
             fdm.ready = nd.ready = false;
         }
         ensure_amg(st);
