@@ -17,7 +17,7 @@ HDRS = [os.path.join(REF, "higtree", "src"), os.path.join(REF, "higflow", "src")
         os.path.join(CONDA, "include"), os.path.join(CONDA, "include", "glib-2.0"),
         os.path.join(CONDA, "lib", "glib-2.0", "include")]
 
-needs = pytest.mark.skipif(not (os.path.isdir(REF) and os.path.exists(os.path.join(CONDA, "include", "mpi.h"))
+needs = pytest.mark.skipif(not (os.path.isfile(os.path.join(HDRS[0], "solver.h")) and os.path.exists(os.path.join(CONDA, "include", "mpi.h"))
                                 and shutil.which("gcc")),
                            reason="reference headers or the MPI/glib headers they include are absent")
 
