@@ -29,8 +29,9 @@ PEAK_HBM_GBS = 8000.0  # MI355X HBM3E
 # the batched sweep of 64 Oldroyd-B cavities (1.2 M cells).  The 2D
 # Oldroyd-B planar 4:1 contraction on its 3-level HiG-Tree AMR mesh and the
 # cavities are smaller cases of the same step.  `roof` names the kernel the
-# roofline line reports: the one that dominates the workload's kernel trace,
-# as (hfh_probe id, name, form probed).
+# roofline line reports, as (hfh_probe id, name, form probed): a launch of the
+# V-cycle that the Krylov solves run on; where the step solves directly, the
+# probe builds that hierarchy first.
 WORKLOADS = {
     # channel of length 20, half-width 4 -> 1, base cells 0.1, 3 factor-2
     # levels within 1.0 of the re-entrant corners (47,800 leaves), parabolic

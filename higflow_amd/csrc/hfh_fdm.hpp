@@ -600,6 +600,7 @@ __global__ void k_fdm_unit(const FdmPin *__restrict__ pins, int n, double *x) {
 class FdmSolver {
   public:
     bool ready = false;
+    bool kronecker = false;  // the matrix has the form (also when the plan was not wanted)
     int n = 0, nd = 0, nsys = 0;
     bool small = false;  // every system fits one workgroup (pass_small)
 
@@ -608,7 +609,7 @@ class FdmSolver {
     // of the diagonal
     bool build(const std::vector<int> &rp, const std::vector<int> &ci, const std::vector<double> &v,
                const std::vector<int> &seg, hipStream_t st, double min_coupling = 0) {
-        ready = false;
+        ready = kronecker = false;
         double coupling = 0;
         n = (int)rp.size() - 1;
         nsys = (int)seg.size() - 1;
@@ -623,6 +624,7 @@ class FdmSolver {
             nd = d;
             for (int e = 0; e < d; e++) coupling = std::max(coupling, std::fabs(sy[q].b[e]) / sy[q].a);
         }
+        kronecker = true;
         if (coupling < min_coupling) return false;
         // the distinct one-dimensional matrices: V, then V^T
         std::map<std::tuple<int, int, int>, std::pair<long, std::vector<double>>> mat;

@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(BLOCK) k_interp_l(int nrow, int ncomp, const i
 // the butterfly order of k_interp_l with L lanes, L = 1 onto the constant as
 // k_interp does, so its value is theirs.  The momentum rows of the 64-cavity
 // sweep (17 M rows of 15 entries), bound before by per-lane template reads
-// and by the uncoalesced entries of the other rows: 670 -> 300 us (1.3 TB/s of writes and column-by-column entries); 256^2 cavity
+// and by the uncoalesced entries of the other rows: 670 -> 300 us; 256^2 cavity
 // 34 -> 23 us, graded contraction 68 -> 42 us, 3D wall layer 424 -> 250 us.
 //
 // Long rows (3D least squares, about 100 entries) take LG lanes per row

@@ -714,7 +714,8 @@ class DeviceSystem {
             std::vector<int> so = seg_off;
             const bool on = direct_allowed();
             fdm.ready = on && fdm.build(hrp, hci, hv, so, st, fdm_min_coupling);
-            nd.ready = on && !fdm.ready && nd_max_flops > 0 && nd.build(hrp, hci, hv, st, nd_max_flops, 2.5e8);
+            // a uniform mesh whose system is left to Jacobi-PCG gets no factors
+            nd.ready = on && !fdm.kronecker && nd_max_flops > 0 && nd.build(hrp, hci, hv, st, nd_max_flops, 2.5e8);
             if (const char *ev = std::getenv("HFH_VERBOSE"))
                 if (std::strcmp(ev, "1") == 0 && (nd_max_flops > 0 || fdm.ready))
                     std::fprintf(stderr, "hfh: system of %d rows: %s (factors %.2g operations, %.2g entries)\n", n,

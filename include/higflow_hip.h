@@ -64,7 +64,9 @@ int hfh_slv_impose_value(hfh_slv *s, int line, double value);
 int hfh_slv_assemble_matrix(hfh_slv *s);
 int hfh_slv_assemble_rhs(hfh_slv *s);
 int hfh_slv_assemble_output(hfh_slv *s);
-/* _solver_vtable.solve (solver.h:55): BiCGStab (right Jacobi) on the device */
+/* _solver_vtable.solve (solver.h:55): BiCGStab (right Jacobi) on the device,
+ * or a direct solve when the matrix is the Kronecker sum of a uniform mesh
+ * (its passes are the iterations that hfh_slv_iterations reports) */
 int hfh_slv_solve(hfh_slv *s);
 /* _solver_vtable.destroy (solver.h:56) */
 void hfh_slv_destroy(hfh_slv *s);
@@ -192,7 +194,8 @@ int hfh_last_solve(hfh_solver *s, int *iters, double *resid, int *outer);
  * converged (higtree/src/solver.h:80-82): info = {iterations, refinement
  * steps, mixed form's FP64 use (0 FP32 refinement, 1 FP32 failed and the
  * solve finished in FP64, 2 FP64 chosen as the faster form), true-residual
- * restarts}; returns 1 converged, 0 not converged, <0 error */
+ * restarts}; a direct solve reports its passes (1 to 4) as iterations;
+ * returns 1 converged, 0 not converged, <0 error */
 int hfh_solve_stats(hfh_solver *s, int which, int *info, double *resid);
 
 /* sd_get_stencil / sfd_get_stencil on the library's host mesh: domain 0

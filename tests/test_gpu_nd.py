@@ -67,3 +67,15 @@ def test_velocity_blocks_of_a_large_mixed_run(monkeypatch):
     x, y = a.get(3, 0), b.get(3, 0)
     assert np.linalg.norm(x - y) <= _cond(a, 1) * (sa["resid"] + sb["resid"]) * np.linalg.norm(y)
     assert not a.get(3, 1).any() and not b.get(3, 1).any()
+
+
+def test_uniform_mesh_with_weak_coupling_keeps_jacobi_pcg():
+    # dt / (Re h^2) = 0.0065: no direct solve, and no factors either
+    case = cases.cavity(256, Re=1000.0, dt=1e-4, tempdiscrtype=cases.SEMI_IMPLICIT_EULER, rtol=RTOL, atol=0.0, maxit=1000)
+    a = native.Flow(case, precision=0)
+    b = native.Flow(case, precision=1, inner_rtol=1e-5)
+    a.step()
+    b.step()
+    # a first solve of the mixed form is the FP64 one: the same iterations
+    assert a.solve_stats(1)["iters"] == b.solve_stats(1)["iters"] > 1
+    assert np.array_equal(a.get(3, 0), b.get(3, 0))
