@@ -269,6 +269,28 @@ int hfh_slv_iterations(hfh_slv *s) { return s ? s->st.iters : fail("null solver"
 double hfh_slv_residual(hfh_slv *s) { return s ? s->st.resid : -1.0; }
 int hfh_slv_converged(hfh_slv *s) { return s ? s->st.converged : fail("null solver"); }
 
+int hfh_direct_plan(int n, const int *rowptr, const int *col, const double *val, double max_ops, double *entries) {
+    if (n < 0 || !rowptr || (n > 0 && (!col || !val))) return fail("hfh_direct_plan: null matrix");
+    for (int i = 0; i < n; i++) {
+        if (rowptr[0] != 0 || rowptr[i + 1] < rowptr[i]) return fail("hfh_direct_plan: row pointers out of order");
+        for (int k = rowptr[i]; k < rowptr[i + 1]; k++)
+            if (col[k] < 0 || col[k] >= n) return fail("hfh_direct_plan: column out of range");
+    }
+    return guard([&] {
+        const int nnz = n > 0 ? rowptr[n] : 0;
+        const std::vector<int> rp(rowptr, rowptr + n + 1), ci(col, col + nnz);
+        const std::vector<double> v(val, val + nnz);
+        const hfh::FdmPlan P = hfh::fdm_plan(rp, ci, v, {0, n}, 0.0);
+        if (entries) *entries = (double)P.entries;
+        if (P.wanted) return 1;
+        if (P.kronecker || max_ops <= 0 || nnz == 0) return 0;
+        hfh::NdTree T;
+        T.symbolic(rp, ci, hfh::ND_LEAF);
+        if (entries) *entries = T.entries;
+        return T.affordable(max_ops, hfh::ND_ENTRIES, hfh::ND_FRONT) && T.numeric(rp, ci, v) ? 2 : 0;
+    });
+}
+
 // ----------------------------------------------------------------- step
 struct hfh_solver {
     std::unique_ptr<hfh::FlowBase> f;

@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <cmath>
 #include <map>
+#include <set>
 #include <stdexcept>
 #include <tuple>
 #include <vector>
@@ -85,22 +86,24 @@ inline void fdm_eigen(int n, int s0, int s1, std::vector<double> &cs, std::vecto
         sn[m] = m < 2 * q ? v : -v;
     }
     cs.resize(n);
-    V.assign((size_t)n * n, 0.0);
-    for (int k = 0; k < n; k++) {
-        const long p = p0 + (long)dp * k;
-        cs[k] = 2.0 * sn[(size_t)((2 * p + q) % (4L * q))];  // 2 cos(pi p / q)
+    V.resize((size_t)n * n);
+    std::vector<double> nn(n, 0.0);
+    for (int k = 0; k < n; k++) cs[k] = 2.0 * sn[(size_t)((2L * (p0 + (long)dp * k) + q) % (4L * q))];  // 2 cos(pi p / q)
+    for (int i = 0; i < n; i++) {
         // the vector starts from the left end's condition: sin(t (i + 1)),
         // cos(t (i + 1/2)) or sin(t (i + 1/2)), t = pi p / q
-        double nn = 0;
-        for (int i = 0; i < n; i++) {
-            const long m = s0 == 0 ? 2 * p * (i + 1) : p * (2L * i + 1) + (s0 == 1 ? q : 0);
-            const double v = sn[(size_t)(m % (4L * q))];
+        const long f = s0 == 0 ? 2L * (i + 1) : 2L * i + 1, step = dp * f % (4L * q);
+        long m = (p0 * f + (s0 == 1 ? q : 0)) % (4L * q);
+        for (int k = 0; k < n; k++) {
+            const double v = sn[(size_t)m];
             V[(size_t)i * n + k] = v;
-            nn += v * v;
+            nn[k] += v * v;
+            if ((m += step) >= 4L * q) m -= 4L * q;
         }
-        const double f = 1.0 / std::sqrt(nn);
-        for (int i = 0; i < n; i++) V[(size_t)i * n + k] *= f;
     }
+    for (int k = 0; k < n; k++) nn[k] = 1.0 / std::sqrt(nn[k]);
+    for (int i = 0; i < n; i++)
+        for (int k = 0; k < n; k++) V[(size_t)i * n + k] *= nn[k];
 }
 
 // Reads the Kronecker form of rows [s.off, s.off + s.len) of a CSR matrix;
@@ -265,6 +268,54 @@ inline bool fdm_detect(const std::vector<int> &rp, const std::vector<int> &ci, c
     const bool singular = std::fabs(lo) <= 1e-10 * hi;
     if (singular) return neumann && s.pin >= 0;
     return lo > 1e-10 * hi && s.pin < 0;
+}
+
+// The systems of a matrix, or why there is no plan.  Each distinct line of n
+// cells costs 2 n^2 table entries (V and V^T), which a pass also reads, so
+// thin boxes lose in the end.  A solve of 65,536 rows, directly and with the
+// V-cycle: 0.18 and 1.8 ms as 1024 x 64, 0.31 and 1.8 ms as 4096 x 16, 0.88
+// and 1.26 ms as 8192 x 8 (tables 1 GB, set-up 2.1 s against 0.1), 2.3 and
+// 1.04 ms as 16384 x 4 (4.3 GB, 12 s): sides up to 8192 are taken.  Square
+// boxes gain at any size measured (2048 x 2048 6.6 against 23 ms).  Tables of
+// all lines: two of the longest (2 GB) plus 4 entries per row, what square
+// boxes of all different sides need.
+constexpr int FDM_SIDE = 8192;
+constexpr long FDM_TABLES = 1L << 28;
+struct FdmPlan {
+    std::vector<FdmSys> sys;
+    int nd = 0;
+    bool kronecker = false;  // the matrix has the form (also when the plan was not wanted)
+    bool wanted = false;     // sides, tables and couplings within the limits
+    long entries = 0;        // of the tables
+};
+// segments as DeviceSystem::set_matrix takes them; not wanted when no
+// coupling reaches min_coupling of the diagonal
+inline FdmPlan fdm_plan(const std::vector<int> &rp, const std::vector<int> &ci, const std::vector<double> &v,
+                        const std::vector<int> &seg, double min_coupling) {
+    FdmPlan P;
+    const int n = (int)rp.size() - 1, nsys = (int)seg.size() - 1;
+    if (n <= 0 || nsys <= 0) return P;
+    P.sys.resize(nsys);
+    double coupling = 0;
+    int side = 0;
+    std::set<std::tuple<int, int, int>> lines;
+    for (int q = 0; q < nsys; q++) {
+        FdmSys &s = P.sys[q];
+        s.off = seg[q];
+        s.len = seg[q + 1] - seg[q];
+        if (seg[q] % 256 != 0 || !fdm_detect(rp, ci, v, s)) return P;
+        const int d = s.n[2] > 1 ? 3 : 2;
+        if (q > 0 && d != P.nd) return P;
+        P.nd = d;
+        for (int e = 0; e < d; e++) {
+            coupling = std::max(coupling, std::fabs(s.b[e]) / s.a);
+            side = std::max(side, s.n[e]);
+            if (lines.emplace(s.n[e], s.s0[e], s.s1[e]).second) P.entries += 2L * s.n[e] * s.n[e];
+        }
+    }
+    P.kronecker = true;
+    P.wanted = coupling >= min_coupling && side <= FDM_SIDE && P.entries <= FDM_TABLES + 4L * n;
+    return P;
 }
 
 // ---------------------------------------------------------------- device
@@ -604,31 +655,21 @@ class FdmSolver {
     int n = 0, nd = 0, nsys = 0;
     bool small = false;  // every system fits one workgroup (pass_small)
 
-    // segments as DeviceSystem::set_matrix takes them; false (no plan) when
-    // a segment has no Kronecker form, or no coupling reaches min_coupling
-    // of the diagonal
+    // false: no plan (fdm_plan)
     bool build(const std::vector<int> &rp, const std::vector<int> &ci, const std::vector<double> &v,
                const std::vector<int> &seg, hipStream_t st, double min_coupling = 0) {
-        ready = kronecker = false;
-        double coupling = 0;
+        ready = false;
+        const FdmPlan plan = fdm_plan(rp, ci, v, seg, min_coupling);
+        kronecker = plan.kronecker;
+        if (!plan.wanted) return false;
         n = (int)rp.size() - 1;
-        nsys = (int)seg.size() - 1;
-        if (n <= 0 || nsys <= 0) return false;
-        std::vector<FdmSys> sy(nsys);
-        for (int q = 0; q < nsys; q++) {
-            sy[q].off = seg[q];
-            sy[q].len = seg[q + 1] - seg[q];
-            if (seg[q] % 256 != 0 || !fdm_detect(rp, ci, v, sy[q])) return false;
-            const int d = sy[q].n[2] > 1 ? 3 : 2;
-            if (q > 0 && d != nd) return false;
-            nd = d;
-            for (int e = 0; e < d; e++) coupling = std::max(coupling, std::fabs(sy[q].b[e]) / sy[q].a);
-        }
-        kronecker = true;
-        if (coupling < min_coupling) return false;
+        nsys = (int)plan.sys.size();
+        nd = plan.nd;
+        const std::vector<FdmSys> &sy = plan.sys;
         // the distinct one-dimensional matrices: V, then V^T
         std::map<std::tuple<int, int, int>, std::pair<long, std::vector<double>>> mat;
         std::vector<double> pool, lam;
+        pool.reserve(plan.entries);
         auto matrix = [&](const FdmSys &s, int d) -> std::pair<long, std::vector<double>> & {
             const auto key = std::make_tuple(s.n[d], s.s0[d], s.s1[d]);
             auto it = mat.find(key);
@@ -638,8 +679,13 @@ class FdmSolver {
                 fdm_eigen(m, s.s0[d], s.s1[d], cs, V);
                 const long at = (long)pool.size();
                 pool.insert(pool.end(), V.begin(), V.end());
-                for (int k = 0; k < m; k++)
-                    for (int i = 0; i < m; i++) pool.push_back(V[(size_t)i * m + k]);
+                pool.resize(pool.size() + V.size());
+                double *T = pool.data() + at + V.size();
+                constexpr int B = 32;  // transposed by blocks
+                for (int i0 = 0; i0 < m; i0 += B)
+                    for (int k0 = 0; k0 < m; k0 += B)
+                        for (int k = k0; k < std::min(m, k0 + B); k++)
+                            for (int i = i0; i < std::min(m, i0 + B); i++) T[(size_t)k * m + i] = V[(size_t)i * m + k];
                 it = mat.emplace(key, std::make_pair(at, cs)).first;
             }
             return it->second;

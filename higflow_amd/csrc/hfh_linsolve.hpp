@@ -715,7 +715,7 @@ class DeviceSystem {
             const bool on = direct_allowed();
             fdm.ready = on && fdm.build(hrp, hci, hv, so, st, fdm_min_coupling);
             // a uniform mesh whose system is left to Jacobi-PCG gets no factors
-            nd.ready = on && !fdm.kronecker && nd_max_flops > 0 && nd.build(hrp, hci, hv, st, nd_max_flops, 2.5e8);
+            nd.ready = on && !fdm.kronecker && nd_max_flops > 0 && nd.build(hrp, hci, hv, st, nd_max_flops, ND_ENTRIES);
             if (const char *ev = std::getenv("HFH_VERBOSE"))
                 if (std::strcmp(ev, "1") == 0 && (nd_max_flops > 0 || fdm.ready))
                     std::fprintf(stderr, "hfh: system of %d rows: %s (factors %.2g operations, %.2g entries)\n", n,

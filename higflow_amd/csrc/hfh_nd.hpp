@@ -233,6 +233,15 @@ class NdTree {
         }
     }
 
+    // whether the factors are within the limits: operations, entries, and
+    // the rows and columns of the largest front
+    bool affordable(double max_flops, double max_entries, int max_front) const {
+        if (flops > max_flops || entries > max_entries) return false;
+        for (const NdNode &N : nodes)
+            if ((int)(N.piv.size() + N.border.size()) > max_front) return false;
+        return true;
+    }
+
     // the factors; false when a front's pivot block is singular
     bool numeric(const std::vector<int> &rp, const std::vector<int> &ci, const std::vector<double> &v) {
         const int n = (int)rp.size() - 1;
@@ -434,6 +443,9 @@ struct NdTask {
 constexpr int ND_NT = 256;
 constexpr int ND_LDS = 8192;  // front entries held in LDS (64 KiB)
 constexpr int ND_PRE = 16;    // matrix entries per lane in flight before the gather
+constexpr int ND_FRONT = ND_LDS - ND_NT / 8;  // the largest front
+constexpr int ND_LEAF = 96;                   // unknowns of a leaf
+constexpr double ND_ENTRIES = 2.5e8;          // of all factors (2 GB)
 // lanes per row: enough that the whole row is in flight (up to 1024 entries)
 inline int nd_lanes(int len) { return len <= 8 * ND_PRE ? 8 : len <= 16 * ND_PRE ? 16 : 64; }
 
@@ -551,13 +563,10 @@ class NdSolver {
         const int n = (int)rp.size() - 1;
         if (n <= 0 || ci.empty()) return false;
         NdTree T;
-        T.symbolic(rp, ci, 96);
+        T.symbolic(rp, ci, ND_LEAF);
         flops = T.flops;
         entries = T.entries;
-        if (T.flops > max_flops || T.entries > max_entries) return false;
-        for (const NdNode &N : T.nodes)
-            if ((int)(N.piv.size() + N.border.size()) > ND_LDS - ND_NT / 8) return false;
-        if (!T.numeric(rp, ci, v)) return false;
+        if (!T.affordable(max_flops, max_entries, ND_FRONT) || !T.numeric(rp, ci, v)) return false;
         const int nn = (int)T.nodes.size();
         std::vector<int> piv, border, sptr(1, 0), src, bo(nn, 0);
         std::vector<double> fac;

@@ -99,6 +99,7 @@ def load():
     L.hfh_slv_residual.argtypes = [vp]
     L.hfh_slv_residual.restype = C.c_double
     L.hfh_slv_set_tolerances.argtypes = [vp, C.c_double, C.c_double, C.c_int]
+    L.hfh_direct_plan.argtypes = [C.c_int, ip, ip, dp, C.c_double, dp]
     L.hfh_create.restype = vp
     L.hfh_create.argtypes = [C.c_int]
     L.hfh_destroy.argtypes = [vp]
@@ -164,6 +165,20 @@ def _check(L, rc, what):
     if rc < 0:
         raise HipError("%s failed (%d): %s" % (what, rc, L.hfh_last_error().decode()))
     return rc
+
+
+def direct_plan(rowptr, cols, vals, max_ops=0.0):
+    """The direct solve a CSR matrix gets: None, "fdm" (fast diagonalisation)
+    or "nd" (nested dissection, its factors within max_ops operations), and
+    the entries of its tables or factors.  Host work only."""
+    L = load()
+    rp = np.ascontiguousarray(rowptr, dtype=np.int32)
+    ci = np.ascontiguousarray(cols, dtype=np.int32)
+    v = np.ascontiguousarray(vals, dtype=np.float64)
+    e = C.c_double()
+    rc = L.hfh_direct_plan(len(rp) - 1, _ip(rp), _ip(ci), _dp(v), float(max_ops), C.byref(e))
+    _check(L, rc, "hfh_direct_plan")
+    return (None, "fdm", "nd")[rc], e.value
 
 
 def params_from(case_params, **over):

@@ -70,6 +70,13 @@ int hfh_slv_assemble_output(hfh_slv *s);
 int hfh_slv_solve(hfh_slv *s);
 /* _solver_vtable.destroy (solver.h:56) */
 void hfh_slv_destroy(hfh_slv *s);
+
+/* The direct solve that an assembled matrix (CSR) gets: 0 none (Krylov),
+ * 1 fast diagonalisation, 2 nested dissection with at most max_ops
+ * operations for its factors (0: not considered, as in the engine).
+ * *entries (may be null): the numbers that its tables or factors hold, or
+ * would hold.  Host work only; needs no device. */
+int hfh_direct_plan(int n, const int *rowptr, const int *col, const double *val, double max_ops, double *entries);
 /* tolerances as slv_set_rel_tol/slv_set_abs_tol/slv_set_maxiteration */
 int hfh_slv_set_tolerances(hfh_slv *s, double rtol, double atol, int maxit);
 /* post-solve fields (solver.h:80-82) */
