@@ -287,7 +287,11 @@ int hfh_direct_plan(int n, const int *rowptr, const int *col, const double *val,
         hfh::NdTree T;
         T.symbolic(rp, ci, hfh::ND_LEAF);
         if (entries) *entries = T.entries;
-        return T.affordable(max_ops, hfh::ND_ENTRIES, hfh::ND_FRONT) && T.numeric(rp, ci, v) ? 2 : 0;
+        try {
+            return T.affordable(max_ops, hfh::ND_ENTRIES, hfh::ND_FRONT) && T.numeric(rp, ci, v) ? 2 : 0;
+        } catch (const std::exception &) {  // the set-up goes on without factors
+            return 0;
+        }
     });
 }
 

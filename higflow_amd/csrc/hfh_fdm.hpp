@@ -790,6 +790,15 @@ class FdmSolver {
         return true;
     }
 
+    void release() {
+        ready = false;
+        small_.free();
+        for (auto &t : tiles_) t.free();
+        jobs_.free();
+        pins_.free();
+        for (KBuf<double> *b : {&mats_, &lam_, &t0_, &t1_, &g_}) b->free();
+    }
+
     // x += M r; psum: sums of r over each 256-row block
     void correct(const double *r, double *x, const double *psum, const double *dinv, hipStream_t st) {
         stages(r, x, psum, dinv, st, true);

@@ -782,15 +782,17 @@ struct KBuf {
     size_t n = 0;
     void alloc(size_t k) {
         if (k <= n && p) return;
-        if (p) (void)hipFree(p);
-        p = nullptr;
+        free();
         if (k == 0) k = 1;
         if (hipMalloc((void **)&p, k * sizeof(T)) != hipSuccess) throw std::runtime_error("hipMalloc failed");
         n = k;
     }
-    ~KBuf() {
+    void free() {
         if (p) (void)hipFree(p);
+        p = nullptr;
+        n = 0;
     }
+    ~KBuf() { free(); }
 };
 
 }  // namespace hfh

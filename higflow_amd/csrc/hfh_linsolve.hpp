@@ -713,9 +713,10 @@ class DeviceSystem {
         {
             std::vector<int> so = seg_off;
             const bool on = direct_allowed();
-            fdm.ready = on && fdm.build(hrp, hci, hv, so, st, fdm_min_coupling);
+            fdm.ready = on && affordable(fdm, [&] { return fdm.build(hrp, hci, hv, so, st, fdm_min_coupling); });
             // a uniform mesh whose system is left to Jacobi-PCG gets no factors
-            nd.ready = on && !fdm.kronecker && nd_max_flops > 0 && nd.build(hrp, hci, hv, st, nd_max_flops, ND_ENTRIES);
+            nd.ready = on && !fdm.kronecker && nd_max_flops > 0 &&
+                       affordable(nd, [&] { return nd.build(hrp, hci, hv, st, nd_max_flops, ND_ENTRIES); });
             if (const char *ev = std::getenv("HFH_VERBOSE"))
                 if (std::strcmp(ev, "1") == 0 && (nd_max_flops > 0 || fdm.ready))
                     std::fprintf(stderr, "hfh: system of %d rows: %s (factors %.2g operations, %.2g entries)\n", n,
@@ -819,6 +820,18 @@ class DeviceSystem {
         return used;
     }
 
+    // a direct solver's set-up; one that runs out of host or device memory
+    // is given back whole and leaves the system to the Krylov solver
+    template <typename S, typename F>
+    static bool affordable(S &solver, F &&build) {
+        try {
+            return build();
+        } catch (const std::exception &) {
+            solver.release();
+            (void)hipGetLastError();
+            return false;
+        }
+    }
     // A run that names a form of the Krylov or V-cycle kernels by one of
     // their switches gets these kernels; HFH_DIRECT=0 turns the direct solves off
     static bool direct_allowed() {

@@ -23,11 +23,11 @@
 #include <atomic>
 #include <cmath>
 #include <stdexcept>
-#include <thread>
 #include <vector>
 
 #include "hfh_krylov.hpp"
 #include "hfh_domain.hpp"
+#include "hfh_parallel.hpp"
 #include "hfh_progress.hpp"
 
 namespace hfh {
@@ -101,13 +101,9 @@ inline void nd_gemm(int nt, int m, int n, int k, double f, const double *A, int 
     if (nt <= 1 || (double)m * n * k < 4e6) return rows(0, m);
     const int step = std::max(16, (m + 4 * nt - 1) / (4 * nt) / 4 * 4);
     std::atomic<int> next{0};
-    auto work = [&] {
+    run_parallel(nt, [&](int) {
         for (int i; (i = next.fetch_add(step)) < m;) rows(i, std::min(m, i + step));
-    };
-    std::vector<std::thread> th;
-    for (int t = 1; t < nt; t++) th.emplace_back(work);
-    work();
-    for (auto &t : th) t.join();
+    });
 }
 
 // inverse of the p x p matrix M (destroyed) into R; false when a pivot
@@ -282,15 +278,19 @@ class NdTree {
                 if (!front(nodes[list[big++]], rp, ci, v, tp, tr, tv, pos[0], nt)) return false;
             }
             std::atomic<size_t> next{big};
-            auto work = [&](int t) {
+            run_parallel(std::min<int>(nt, (int)list.size()), [&](int t) {
+                struct Stop {  // the others end with the first that does not return
+                    std::atomic<bool> &ok;
+                    bool done = false;
+                    ~Stop() {
+                        if (!done) ok = false;
+                    }
+                } stop{ok};
                 if (pos[t].empty()) pos[t].assign(n, -1);
                 for (size_t i; ok && (i = next++) < list.size();)
                     if (!front(nodes[list[i]], rp, ci, v, tp, tr, tv, pos[t], 1)) ok = false;
-            };
-            std::vector<std::thread> th;
-            for (int t = 1; t < std::min<int>(nt, (int)list.size()); t++) th.emplace_back(work, t);
-            work(0);
-            for (auto &t : th) t.join();
+                stop.done = true;
+            });
             if (!ok) return false;
         }
         return true;
@@ -649,6 +649,14 @@ class NdSolver {
         k_fill<double><<<nblocks(n), BLOCK, 0, st>>>(n, z_.p, 0.0);
         ready = true;
         return true;
+    }
+
+    void release() {
+        ready = false;
+        for (KBuf<int> *b : {&piv_, &border_, &sptr_, &src_}) b->free();
+        ut_.free();
+        dt_.free();
+        for (KBuf<double> *b : {&fac_, &y_, &updv_, &z_}) b->free();
     }
 
     // x += A^-1 r
