@@ -531,7 +531,7 @@ __global__ void __launch_bounds__(FDM_SNT) k_fdm_small(const FdmSmall *__restric
                                                        int nd, KRows<double> A, const double *__restrict__ mats,
                                                        const double *__restrict__ lam, const double *__restrict__ g,
                                                        const double *__restrict__ dinv, const double *__restrict__ b,
-                                                       double *__restrict__ x, double *norms) {
+                                                       double *__restrict__ x, double *__restrict__ bak, double *norms) {
     extern __shared__ double fdm_lds[];
     __shared__ double sh[3][FDM_SNT / 64];
     __shared__ double s_rp;
@@ -601,7 +601,8 @@ __global__ void __launch_bounds__(FDM_SNT) k_fdm_small(const FdmSmall *__restric
     fdm_small_stage<0>(J, Z[0], w, [&](int m, int n, int, int, double z) {
         const int i = m * nx + n, gi = J.off + i;
         if (P.pin >= 0) z = i == P.pin ? zp : z + (mu * g[gi] + c);
-        const double xn = x[gi] + z;
+        const double x0 = x[gi], xn = x0 + z;
+        bak[gi] = x0;
         x[gi] = xn;
         u[i] = xn;
     });
@@ -804,11 +805,12 @@ class FdmSolver {
         stages(r, x, psum, dinv, st, true);
     }
 
-    // x += M (b - A x) and the norms of the new residual and of b, with one
-    // workgroup per system
-    void pass_small(const KRows<double> &A, const double *dinv, const double *b, double *x, double *norms,
+    // x += M (b - A x), the x before in bak, and the norms of the new
+    // residual and of b, with one workgroup per system
+    void pass_small(const KRows<double> &A, const double *dinv, const double *b, double *x, double *bak, double *norms,
                     hipStream_t st) {
-        k_fdm_small<<<nsys, FDM_SNT, small_lds_, st>>>(small_.p, pins_.p, nd, A, mats_.p, lam_.p, g_.p, dinv, b, x, norms);
+        k_fdm_small<<<nsys, FDM_SNT, small_lds_, st>>>(small_.p, pins_.p, nd, A, mats_.p, lam_.p, g_.p, dinv, b, x, bak,
+                                                       norms);
     }
 
   private:

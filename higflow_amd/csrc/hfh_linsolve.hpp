@@ -351,7 +351,7 @@ __global__ void __launch_bounds__(BLOCK) k_residual(int n, const int *__restrict
 
 // the same with 4 lanes per row: workgroups of 4 BLOCK threads, one per
 // BLOCK rows, so the partials have k_residual's layout (one per BLOCK rows);
-// prs: the sums of r.  LG = 16 takes the rows in four turns of 16 lanes: the
+// prs: the sums of r; xcopy (if given): a copy of x.  LG = 16 takes the rows in four turns of 16 lanes: the
 // least-squares rows of a 3D mesh (30-65 entries on average, up to 200) wait
 // for their longest row, 49 us on 4 lanes for 47,592 rows, 36 us on 16.
 template <typename T, int LG = 4>
@@ -359,7 +359,8 @@ __global__ void __launch_bounds__(4 * BLOCK) k_residual_l4(int n, const int *__r
                                                            const int *__restrict__ ci, const T *__restrict__ v,
                                                            const T *__restrict__ x, const T *__restrict__ b,
                                                            T *__restrict__ r, T *__restrict__ prr,
-                                                           T *__restrict__ pbb, T *__restrict__ prs) {
+                                                           T *__restrict__ pbb, T *__restrict__ prs,
+                                                           T *__restrict__ xcopy) {
     const int lane = threadIdx.x % LG;
     T rr = 0, bb = 0, rs = 0;
 #pragma unroll
@@ -373,6 +374,7 @@ __global__ void __launch_bounds__(4 * BLOCK) k_residual_l4(int n, const int *__r
         if (i < n && lane == 0) {
             const T bi = b[i], ri = bi - s;
             r[i] = ri;
+            if (xcopy) xcopy[i] = x[i];
             rr += ri * ri;
             bb += bi * bi;
             rs += ri;
@@ -409,7 +411,8 @@ __global__ void __launch_bounds__(4 * BLOCK) k_residual_l4(int n, const int *__r
 template <typename T>
 __global__ void __launch_bounds__(KNT) k_residual_d(int n, KRows<T> A, const T *__restrict__ x,
                                                     const T *__restrict__ b, T *__restrict__ r, T *__restrict__ prr,
-                                                    T *__restrict__ pbb, T *__restrict__ prs, int nb) {
+                                                    T *__restrict__ pbb, T *__restrict__ prs, int nb,
+                                                    T *__restrict__ xcopy) {
     const int i = blockIdx.x * KNT + (int)threadIdx.x;
     const bool in = i < n;
     const int *db = A.dblk + (size_t)blockIdx.x * (KD_MAX + 1);
@@ -438,6 +441,7 @@ __global__ void __launch_bounds__(KNT) k_residual_d(int n, KRows<T> A, const T *
     if (in) {
         const T bi = b[i], ri = bi - s;
         r[i] = ri;
+        if (xcopy) xcopy[i] = x[i];
         rr = ri * ri;
         bb = bi * bi;
         rs = ri;
@@ -468,6 +472,15 @@ __global__ void __launch_bounds__(KNT) k_residual_d(int n, KRows<T> A, const T *
             prs[pb] = e;
         }
     }
+}
+
+// dst = src in the segments whose flag is set (bseg: segment of each BLOCK
+// rows, null for one segment), in the rows that have entries
+__global__ void __launch_bounds__(BLOCK) k_seg_copy(int n, const int *__restrict__ rp, const int *__restrict__ bseg,
+                                                    const int *flag, const double *__restrict__ src,
+                                                    double *__restrict__ dst) {
+    const int i = blockIdx.x * BLOCK + (int)threadIdx.x;
+    if (i < n && flag[bseg ? bseg[blockIdx.x] : 0] && rp[i + 1] > rp[i]) dst[i] = src[i];
 }
 
 template <typename T>
@@ -661,7 +674,8 @@ class DeviceSystem {
         off_sc_ = off_ks_ + ((nseg * KS_N * (int)sizeof(double) + 63) / 64) * 64;
         off_rr_ = off_sc_ + 256;
         off_fd_ = off_rr_ + 2 * nb * (int)sizeof(double);
-        const size_t pin = (size_t)off_fd_ + 2 * (size_t)nseg * sizeof(double);
+        off_bk_ = off_fd_ + 2 * nseg * (int)sizeof(double);
+        const size_t pin = (size_t)off_bk_ + (size_t)nseg * sizeof(int);
         clear_graphs();
         {
             // off by default: on the 64-cavity sweep the graph took the FP64
@@ -856,20 +870,31 @@ class DeviceSystem {
         hv_.clear();
     }
 
-    // Direct solve (hfh_fdm.hpp, hfh_nd.hpp): x += M (b - A x) until the true residual
-    // passes the stopping test or stops falling.  False when the corrections
-    // do not converge (the caller goes on with the Krylov solver from x).
-    bool direct_solve(const double *b, double *x, double rtol, double atol, hipStream_t st, SolveStats &S) {
+    // Direct solve (hfh_fdm.hpp, hfh_nd.hpp): x += M (b - A x) until the true
+    // residual passes the stopping test or stops falling.  Every segment is
+    // judged by itself: one that has ended keeps its x while the others go
+    // on.  False when a segment is left to the Krylov solver (SEG_KRYLOV in
+    // seg_state_), from its best x; a correction that is not finite is undone.
+    enum { SEG_OPEN = 0, SEG_FINAL, SEG_KRYLOV };
+    bool direct_solve(const double *b, double *x, double rtol, double atol, int fallback, hipStream_t st, SolveStats &S) {
         double *norms = reinterpret_cast<double *>(hpin_ + off_fd_);
+        int *back = reinterpret_cast<int *>(hpin_ + off_bk_);
         const double *h = norms;
-        std::vector<SolveStats> gs(nseg);
-        double best = -1.0;
+        std::vector<SolveStats> &gs = seg_stats;
+        S = SolveStats();
+        S.fallback = fallback;
+        gs.assign(nseg, S);
+        seg_state_.assign(nseg, SEG_OPEN);
+        bool open = true, undone = false, bad = false;
         const bool small = fdm.ready && fdm.small;
-        if (!small) true_residual(x, b, st);
-        for (int pass = 1; pass <= 4; pass++) {
-            if (pass > 1) HFH_CHECK(hipMemcpyAsync(xbak.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
+        if (!small) true_residual(x, b, st, xbak.p);
+        int pass = 0;
+        while (open && pass < 4) {
+            pass++;
+            if (pass > 1 && !small)
+                HFH_CHECK(hipMemcpyAsync(xbak.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
             if (small) {
-                fdm.pass_small(k64.Av, dinv.p, b, x, norms, st);
+                fdm.pass_small(k64.Av, dinv.p, b, x, xbak.p, norms, st);
             } else {
                 if (fdm.ready)
                     fdm.correct(r.p, x, part3.p, dinv.p, st);
@@ -879,67 +904,135 @@ class DeviceSystem {
                 k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part2.p, norms);
             }
             if (pass == 1 && early) early();
-            early_done = pass == 1 && early;
             HFH_CHECK(hipStreamSynchronize(st));
-            bool all_conv = true;
-            double worst = 0;
+            open = false;
+            bool undo = false;
             for (int g = 0; g < nseg; g++) {
                 const double rn = std::sqrt(h[2 * g]), bn = std::sqrt(h[2 * g + 1]), tol = std::max(rtol * bn, atol);
-                gs[g].iters = pass;
-                gs[g].resid = bn > 0 ? rn / bn : rn;
-                gs[g].converged = rn <= tol;
-                all_conv = all_conv && gs[g].converged;
-                worst = std::isfinite(gs[g].resid) ? std::max(worst, gs[g].resid) : gs[g].resid;
-                if (!std::isfinite(worst)) break;
+                const double resid = bn > 0 ? rn / bn : rn, old = gs[g].resid;
+                const bool better = seg_state_[g] == SEG_OPEN && std::isfinite(rn) && (pass == 1 || resid < old);
+                back[g] = !better;
+                undo = undo || !better;
+                if (better) {
+                    gs[g].iters = pass;
+                    gs[g].resid = resid;
+                    gs[g].converged = rn <= tol;
+                }
+                if (seg_state_[g] != SEG_OPEN) continue;
+                if (gs[g].converged) {
+                    seg_state_[g] = SEG_FINAL;
+                } else if (pass == 1 && !better) {
+                    seg_state_[g] = SEG_KRYLOV;
+                    bad = true;
+                } else if (pass > 1 && !(resid < 0.5 * old)) {
+                    // a correction that no longer halves the residual has
+                    // reached its rounding (b - A x carries eps |A| |x|), where
+                    // the Krylov solver has nothing to add
+                    seg_state_[g] = gs[g].resid < 1e-8 ? SEG_FINAL : SEG_KRYLOV;
+                } else {
+                    open = true;
+                }
             }
-            S.iters = pass;
-            if (!std::isfinite(worst)) {
-                all_conv = false;
-                if (pass == 1) return false;
+            if (undo) {
+                k_seg_copy<<<nb, BLOCK, 0, st>>>(n, rp.p, nseg > 1 ? bseg_.p : nullptr, back, xbak.p, x);
+                undone = true;
             }
-            const bool better = pass == 1 || worst < best;
-            if (!better) {
-                HFH_CHECK(hipMemcpyAsync(x, xbak.p, n * sizeof(double), hipMemcpyDeviceToDevice, st));
-            } else {
-                seg_stats = gs;
-                S.resid = worst;
-                S.converged = all_conv;
-            }
-            if (all_conv) return true;
-            // a correction that no longer halves the residual has reached its
-            // rounding (b - A x carries eps |A| |x|)
-            if (pass > 1 && !(worst < 0.5 * best)) break;
-            best = worst;
         }
-        // at the rounding of the residual the Krylov solver has nothing to add
-        return S.resid < 1e-8;
+        for (int g = 0; g < nseg; g++)
+            if (seg_state_[g] == SEG_OPEN) seg_state_[g] = gs[g].resid < 1e-8 ? SEG_FINAL : SEG_KRYLOV;
+        if (bad) {
+            // where the residual was not finite to begin with, x stays what
+            // it was: the Krylov solver would leave it, too
+            true_residual(x, b, st);
+            k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part2.p, norms);
+            HFH_CHECK(hipStreamSynchronize(st));
+            for (int g = 0; g < nseg; g++) {
+                const double rn = std::sqrt(h[2 * g]), bn = std::sqrt(h[2 * g + 1]);
+                if (gs[g].iters > 0 || std::isfinite(rn)) continue;
+                seg_state_[g] = SEG_FINAL;
+                gs[g].resid = bn > 0 ? rn / bn : rn;
+            }
+        }
+        early_done = early && pass == 1 && !undone;
+        S.iters = pass;
+        return sum_segments(S);
+    }
+    // S's residual and convergence from the segments'; true when all are final
+    bool sum_segments(SolveStats &S) {
+        bool fin = true;
+        S.resid = 0;
+        S.converged = 1;
+        for (int g = 0; g < nseg; g++) {
+            const double q = seg_stats[g].resid;
+            if (!(q <= S.resid) && !std::isnan(S.resid)) S.resid = q;
+            S.converged = S.converged && seg_stats[g].converged;
+            fin = fin && seg_state_[g] == SEG_FINAL;
+        }
+        return fin;
+    }
+
+    // The direct solve, then krylov() for the segments that it leaves: the
+    // others keep their x and statistics.  This solve only: the next one
+    // starts with the direct solve again.  `fallback`: SolveStats::fallback of
+    // what the direct solve ends.
+    template <typename F>
+    SolveStats direct_first(const double *b, double *x, double rtol, double atol, int fallback, hipStream_t st,
+                            F &&krylov) {
+        SolveStats S;
+        if (direct_solve(b, x, rtol, atol, fallback, st, S)) return S;
+        early_done = false;
+        const std::vector<SolveStats> gs = seg_stats;
+        const std::vector<int> state = seg_state_;
+        bool keep = false;
+        for (int q : state) keep = keep || q == SEG_FINAL;
+        if (keep) {
+            if ((int)xkeep_.n < n) xkeep_.alloc(n);
+            HFH_CHECK(hipMemcpyAsync(xkeep_.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
+        }
+        SolveStats K = krylov();
+        K.iters += S.iters;
+        if (nseg == 1) return K;
+        if (keep) {
+            int *back = reinterpret_cast<int *>(hpin_ + off_bk_);
+            for (int g = 0; g < nseg; g++) back[g] = state[g] == SEG_FINAL;
+            k_seg_copy<<<nb, BLOCK, 0, st>>>(n, rp.p, bseg_.p, back, xkeep_.p, x);
+        }
+        for (int g = 0; g < nseg; g++) {
+            if (state[g] == SEG_FINAL)
+                seg_stats[g] = gs[g];
+            else
+                seg_stats[g].iters += S.iters;
+        }
+        sum_segments(K);
+        return K;
     }
 
     // r = b - A x and the per-256-row partials of r.r and b.b in part1 /
     // part2: the diagonal-form rows when the FP64 solver has them
-    // (HFH_RESID_DIAG=0: the CSR launch)
-    void true_residual(const double *x, const double *b, hipStream_t st) {
+    // (HFH_RESID_DIAG=0: the CSR launch); xcopy (if given) = x
+    void true_residual(const double *x, const double *b, hipStream_t st, double *xcopy = nullptr) {
         if (k64.Av.dw && resid_diag_)
             k_residual_d<double><<<(n + KNT - 1) / KNT, KNT, 0, st>>>(n, k64.Av, x, b, r.p, part1.p, part2.p,
-                                                                       part3.p, nb);
+                                                                       part3.p, nb, xcopy);
         else if (nnz > 24L * n)
-            k_residual_l4<double, 16><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p);
+            k_residual_l4<double, 16><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p,
+                                                                xcopy);
         else
-            k_residual_l4<double><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p);
+            k_residual_l4<double><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p,
+                                                            xcopy);
     }
 
     // FP64 fused solve: Jacobi-PCG (spd) or BiCGStab, warm-started from x.
     // The stopping test runs on the recursively updated residual; once it
     // passes, the true residual b - A x is checked and the iteration
     // restarted from x (at most twice) while it misses the tolerance.
+    // Systems with a direct solver try that first.
     SolveStats fused64(bool spd, const double *b, double *x, double rtol, double atol, int maxit, hipStream_t st) {
         early_done = false;
-        if (direct() && maxit > 0) {
-            SolveStats F;
-            if (direct_solve(b, x, rtol, atol, st, F)) return F;
-            early_done = false;
-            fdm.ready = nd.ready = false;
-        }
+        auto krylov = [&] { return krylov64(spd, b, x, rtol, atol, maxit, st); };
+        return direct() && maxit > 0 ? direct_first(b, x, rtol, atol, 0, st, krylov) : krylov();
+    }
+    SolveStats krylov64(bool spd, const double *b, double *x, double rtol, double atol, int maxit, hipStream_t st) {
         ensure_amg(st);
         int hi[KI_N];
         double hs[KS_N];
@@ -1099,16 +1192,12 @@ class DeviceSystem {
     SolveStats fused_mixed(bool spd, const double *b, double *x, double rtol, double atol, double inner_rtol,
                            int maxit, hipStream_t st) {
         early_done = false;
-        if (direct() && maxit > 0) {
-            SolveStats F;
-            if (direct_solve(b, x, rtol, atol, st, F)) {
-                F.fallback = 2;  // FP64 throughout
-                for (auto &g : seg_stats) g.fallback = 2;
-                return F;
-            }
-            early_done = false;
-            fdm.ready = nd.ready = false;
-        }
+        auto krylov = [&] { return krylov_mixed(spd, b, x, rtol, atol, inner_rtol, maxit, st); };
+        // a direct solve is FP64 throughout (fallback 2)
+        return direct() && maxit > 0 ? direct_first(b, x, rtol, atol, 2, st, krylov) : krylov();
+    }
+    SolveStats krylov_mixed(bool spd, const double *b, double *x, double rtol, double atol, double inner_rtol,
+                            int maxit, hipStream_t st) {
         ensure_amg(st);
         account_pending();
         bool use32, probing = false;
@@ -1141,7 +1230,7 @@ class DeviceSystem {
             if (!S.converged && S.fallback == 0) {
                 // the refinement stalled (FP32 too coarse for this system):
                 // finish in FP64 from the current x
-                SolveStats F = fused64(spd, b, x, rtol, atol, maxit, st);
+                SolveStats F = krylov64(spd, b, x, rtol, atol, maxit, st);
                 F.iters += S.iters;
                 F.outer = S.outer;
                 F.fallback = 1;
@@ -1154,7 +1243,7 @@ class DeviceSystem {
             // against 36 with the FP64 cycle) and stop on its updated
             // residual with a wrong x.
             k64.use_amg32 = mixed_amg32_ && spd;
-            S = fused64(spd, b, x, rtol, atol, maxit, st);
+            S = krylov64(spd, b, x, rtol, atol, maxit, st);
             k64.use_amg32 = false;
             S.fallback = 2;
             for (auto &g : seg_stats) g.fallback = 2;
@@ -1283,7 +1372,7 @@ class DeviceSystem {
                 // FP32 Krylov cannot reach inner_rtol on this system (too
                 // ill-conditioned for single precision): finish in FP64 from
                 // the current x (the caller keeps FP64 for a while)
-                SolveStats F = fused64(spd, b, x, rtol, atol, maxit, st);
+                SolveStats F = krylov64(spd, b, x, rtol, atol, maxit, st);
                 F.iters += inner_total;
                 F.outer = outer;
                 F.fallback = 1;
@@ -1466,6 +1555,9 @@ class DeviceSystem {
     char *hpin_ = nullptr;  // pinned status: flags at 0, fused scalars at 64, outer scalars at 256
     int off_rr_ = 512;      // pinned true-residual partials (r.r then b.b, nb each)
     int off_fd_ = 0;        // pinned r.r and b.b per segment (direct solves)
+    int off_bk_ = 0;        // pinned flag per segment: its x is put back
+    std::vector<int> seg_state_;  // of the last direct solve
+    DevBuf<double> xkeep_;        // x of the segments that a direct solve has ended, during a Krylov solve of others
     std::vector<int> hrp_, hci_;  // the matrix, while its hierarchy is deferred
     std::vector<double> hv_;
     bool graph_on_ = false;  // first pass of FP64 fused solves as a captured graph (HFH_GRAPH=1)
