@@ -483,6 +483,35 @@ __global__ void __launch_bounds__(BLOCK) k_seg_copy(int n, const int *__restrict
     if (i < n && flag[bseg ? bseg[blockIdx.x] : 0] && rp[i + 1] > rp[i]) dst[i] = src[i];
 }
 
+// what rounding can leave in the 2-norm of b - A x: partials, per 256-row
+// block, of ((len + 2) u |A||x| + u |b|)^2 (len entries of the row, u = 2^-53;
+// the sum and the difference as evaluated, and x as rounded), 4 lanes per row
+__global__ void __launch_bounds__(4 * BLOCK) k_resid_rounding(int n, const int *__restrict__ rp,
+                                                              const int *__restrict__ ci, const double *__restrict__ v,
+                                                              const double *__restrict__ x,
+                                                              const double *__restrict__ b, double *__restrict__ part) {
+    const int lane = threadIdx.x & 3, i = blockIdx.x * BLOCK + (int)threadIdx.x / 4;
+    double s = 0;
+    if (i < n)
+        for (int k = rp[i] + lane; k < rp[i + 1]; k += 4) s += fabs(v[k] * x[ci[k]]);
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    double e = 0;
+    if (i < n && lane == 0) {
+        e = 0x1p-53 * ((rp[i + 1] - rp[i] + 2) * s + fabs(b[i]));
+        e *= e;
+    }
+    e = wave_sum(e);
+    __shared__ double se[4 * BLOCK / 64];
+    if ((threadIdx.x & 63) == 0) se[threadIdx.x >> 6] = e;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double a = 0;
+        for (int q = 0; q < 4 * BLOCK / 64; q++) a += se[q];
+        part[blockIdx.x] = a;
+    }
+}
+
 template <typename T>
 struct DevBuf {
     T *p = nullptr;
@@ -674,7 +703,7 @@ class DeviceSystem {
         off_sc_ = off_ks_ + ((nseg * KS_N * (int)sizeof(double) + 63) / 64) * 64;
         off_rr_ = off_sc_ + 256;
         off_fd_ = off_rr_ + 2 * nb * (int)sizeof(double);
-        off_bk_ = off_fd_ + 2 * nseg * (int)sizeof(double);
+        off_bk_ = off_fd_ + 4 * nseg * (int)sizeof(double);
         const size_t pin = (size_t)off_bk_ + (size_t)nseg * sizeof(int);
         clear_graphs();
         {
@@ -725,6 +754,8 @@ class DeviceSystem {
         // matrices with a Kronecker form are solved directly; their hierarchy
         // is built when a solve or a probe first needs it
         {
+            const char *ep = std::getenv("HFH_DIRECT_PASSES");
+            direct_passes_ = ep ? std::max(1, std::atoi(ep)) : 4;
             std::vector<int> so = seg_off;
             const bool on = direct_allowed();
             fdm.ready = on && affordable(fdm, [&] { return fdm.build(hrp, hci, hv, so, st, fdm_min_coupling); });
@@ -871,13 +902,16 @@ class DeviceSystem {
     }
 
     // Direct solve (hfh_fdm.hpp, hfh_nd.hpp): x += M (b - A x) until the true
-    // residual passes the stopping test or stops falling.  Every segment is
+    // residual passes the stopping test, or no longer halves and is not above
+    // its own rounding, where no solver has anything to add.  Every segment is
     // judged by itself: one that has ended keeps its x while the others go
     // on.  False when a segment is left to the Krylov solver (SEG_KRYLOV in
-    // seg_state_), from its best x; a correction that is not finite is undone.
+    // seg_state_), from its best x, after at most `limit` passes; a correction
+    // that is not finite is undone.
     enum { SEG_OPEN = 0, SEG_FINAL, SEG_KRYLOV };
-    bool direct_solve(const double *b, double *x, double rtol, double atol, int fallback, hipStream_t st, SolveStats &S) {
-        double *norms = reinterpret_cast<double *>(hpin_ + off_fd_);
+    bool direct_solve(const double *b, double *x, double rtol, double atol, int limit, int fallback, hipStream_t st,
+                      SolveStats &S) {
+        double *norms = reinterpret_cast<double *>(hpin_ + off_fd_), *rounding = norms + 2 * nseg;
         int *back = reinterpret_cast<int *>(hpin_ + off_bk_);
         const double *h = norms;
         std::vector<SolveStats> &gs = seg_stats;
@@ -889,7 +923,7 @@ class DeviceSystem {
         const bool small = fdm.ready && fdm.small;
         if (!small) true_residual(x, b, st, xbak.p);
         int pass = 0;
-        while (open && pass < 4) {
+        while (open && pass < limit) {
             pass++;
             if (pass > 1 && !small)
                 HFH_CHECK(hipMemcpyAsync(xbak.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
@@ -907,6 +941,7 @@ class DeviceSystem {
             HFH_CHECK(hipStreamSynchronize(st));
             open = false;
             bool undo = false;
+            std::vector<int> stalled;
             for (int g = 0; g < nseg; g++) {
                 const double rn = std::sqrt(h[2 * g]), bn = std::sqrt(h[2 * g + 1]), tol = std::max(rtol * bn, atol);
                 const double resid = bn > 0 ? rn / bn : rn, old = gs[g].resid;
@@ -925,21 +960,27 @@ class DeviceSystem {
                     seg_state_[g] = SEG_KRYLOV;
                     bad = true;
                 } else if (pass > 1 && !(resid < 0.5 * old)) {
-                    // a correction that no longer halves the residual has
-                    // reached its rounding (b - A x carries eps |A| |x|), where
-                    // the Krylov solver has nothing to add
-                    seg_state_[g] = gs[g].resid < 1e-8 ? SEG_FINAL : SEG_KRYLOV;
+                    stalled.push_back(g);
                 } else {
                     open = true;
                 }
             }
             if (undo) {
-                k_seg_copy<<<nb, BLOCK, 0, st>>>(n, rp.p, nseg > 1 ? bseg_.p : nullptr, back, xbak.p, x);
+                put_back(xbak.p, x, st);
                 undone = true;
+            }
+            if (!stalled.empty()) {
+                k_resid_rounding<<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, part1.p);
+                k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part1.p, rounding);
+                HFH_CHECK(hipStreamSynchronize(st));
+                for (int g : stalled) {
+                    const double bn = std::sqrt(h[2 * g + 1]), kept = gs[g].resid * (bn > 0 ? bn : 1.0);
+                    seg_state_[g] = kept <= std::sqrt(rounding[2 * g]) ? SEG_FINAL : SEG_KRYLOV;
+                }
             }
         }
         for (int g = 0; g < nseg; g++)
-            if (seg_state_[g] == SEG_OPEN) seg_state_[g] = gs[g].resid < 1e-8 ? SEG_FINAL : SEG_KRYLOV;
+            if (seg_state_[g] == SEG_OPEN) seg_state_[g] = SEG_KRYLOV;
         if (bad) {
             // where the residual was not finite to begin with, x stays what
             // it was: the Krylov solver would leave it, too
@@ -957,6 +998,15 @@ class DeviceSystem {
         S.iters = pass;
         return sum_segments(S);
     }
+    // x = from in the segments flagged at off_bk_ of the pinned status (not
+    // written again before the next wait on the stream).  The flags go to the
+    // device first: read from there by each workgroup, host memory costs more
+    // than the copies.
+    void put_back(const double *from, double *x, hipStream_t st) {
+        if ((int)segback_.n < nseg) segback_.alloc(nseg);
+        HFH_CHECK(hipMemcpyAsync(segback_.p, hpin_ + off_bk_, nseg * sizeof(int), hipMemcpyHostToDevice, st));
+        k_seg_copy<<<nb, BLOCK, 0, st>>>(n, rp.p, nseg > 1 ? bseg_.p : nullptr, segback_.p, from, x);
+    }
     // S's residual and convergence from the segments'; true when all are final
     bool sum_segments(SolveStats &S) {
         bool fin = true;
@@ -971,15 +1021,16 @@ class DeviceSystem {
         return fin;
     }
 
-    // The direct solve, then krylov() for the segments that it leaves: the
-    // others keep their x and statistics.  This solve only: the next one
-    // starts with the direct solve again.  `fallback`: SolveStats::fallback of
-    // what the direct solve ends.
+    // The direct solve, then krylov(iterations left of maxit) for the segments
+    // that it leaves: the others keep their x and statistics.  This solve
+    // only: the next one starts with the direct solve again.  `fallback`:
+    // SolveStats::fallback of what the direct solve ends.
     template <typename F>
-    SolveStats direct_first(const double *b, double *x, double rtol, double atol, int fallback, hipStream_t st,
-                            F &&krylov) {
+    SolveStats direct_first(const double *b, double *x, double rtol, double atol, int maxit, int fallback,
+                            hipStream_t st, F &&krylov) {
         SolveStats S;
-        if (direct_solve(b, x, rtol, atol, fallback, st, S)) return S;
+        const bool done = direct_solve(b, x, rtol, atol, std::min(direct_passes_, maxit), fallback, st, S);
+        if (done || S.iters >= maxit) return S;
         early_done = false;
         const std::vector<SolveStats> gs = seg_stats;
         const std::vector<int> state = seg_state_;
@@ -989,13 +1040,13 @@ class DeviceSystem {
             if ((int)xkeep_.n < n) xkeep_.alloc(n);
             HFH_CHECK(hipMemcpyAsync(xkeep_.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
         }
-        SolveStats K = krylov();
+        SolveStats K = krylov(maxit - S.iters);
         K.iters += S.iters;
         if (nseg == 1) return K;
         if (keep) {
             int *back = reinterpret_cast<int *>(hpin_ + off_bk_);
             for (int g = 0; g < nseg; g++) back[g] = state[g] == SEG_FINAL;
-            k_seg_copy<<<nb, BLOCK, 0, st>>>(n, rp.p, bseg_.p, back, xkeep_.p, x);
+            put_back(xkeep_.p, x, st);
         }
         for (int g = 0; g < nseg; g++) {
             if (state[g] == SEG_FINAL)
@@ -1029,8 +1080,8 @@ class DeviceSystem {
     // Systems with a direct solver try that first.
     SolveStats fused64(bool spd, const double *b, double *x, double rtol, double atol, int maxit, hipStream_t st) {
         early_done = false;
-        auto krylov = [&] { return krylov64(spd, b, x, rtol, atol, maxit, st); };
-        return direct() && maxit > 0 ? direct_first(b, x, rtol, atol, 0, st, krylov) : krylov();
+        auto krylov = [&](int left) { return krylov64(spd, b, x, rtol, atol, left, st); };
+        return direct() && maxit > 0 ? direct_first(b, x, rtol, atol, maxit, 0, st, krylov) : krylov(maxit);
     }
     SolveStats krylov64(bool spd, const double *b, double *x, double rtol, double atol, int maxit, hipStream_t st) {
         ensure_amg(st);
@@ -1192,9 +1243,9 @@ class DeviceSystem {
     SolveStats fused_mixed(bool spd, const double *b, double *x, double rtol, double atol, double inner_rtol,
                            int maxit, hipStream_t st) {
         early_done = false;
-        auto krylov = [&] { return krylov_mixed(spd, b, x, rtol, atol, inner_rtol, maxit, st); };
+        auto krylov = [&](int left) { return krylov_mixed(spd, b, x, rtol, atol, inner_rtol, left, st); };
         // a direct solve is FP64 throughout (fallback 2)
-        return direct() && maxit > 0 ? direct_first(b, x, rtol, atol, 2, st, krylov) : krylov();
+        return direct() && maxit > 0 ? direct_first(b, x, rtol, atol, maxit, 2, st, krylov) : krylov(maxit);
     }
     SolveStats krylov_mixed(bool spd, const double *b, double *x, double rtol, double atol, double inner_rtol,
                             int maxit, hipStream_t st) {
@@ -1554,8 +1605,10 @@ class DeviceSystem {
   private:
     char *hpin_ = nullptr;  // pinned status: flags at 0, fused scalars at 64, outer scalars at 256
     int off_rr_ = 512;      // pinned true-residual partials (r.r then b.b, nb each)
-    int off_fd_ = 0;        // pinned r.r and b.b per segment (direct solves)
+    int off_fd_ = 0;        // pinned r.r and b.b, then their rounding, per segment (direct solves)
+    int direct_passes_ = 4; // of a direct solve (HFH_DIRECT_PASSES)
     int off_bk_ = 0;        // pinned flag per segment: its x is put back
+    DevBuf<int> segback_;         // the same on the device
     std::vector<int> seg_state_;  // of the last direct solve
     DevBuf<double> xkeep_;        // x of the segments that a direct solve has ended, during a Krylov solve of others
     std::vector<int> hrp_, hci_;  // the matrix, while its hierarchy is deferred

@@ -1,6 +1,6 @@
-"""What a direct solve leaves behind when a right-hand side is not finite, or
-when some systems of a batch end before others: the next solves and the other
-systems are, to the bit, what they are without it."""
+"""Direct solves that are not the last word: right-hand sides that are not
+finite, systems of a batch that end before others, passes that run out.  The
+next solves and the other systems are, to the bit, what they are without it."""
 import numpy as np
 import pytest
 
@@ -91,3 +91,80 @@ def test_members_beside_one_that_is_not_finite(sides, dim, precision):
         a.step()
         b.step()
         assert not same(range(3))
+
+
+def _far(nx, ny):
+    """A right-hand side and a guess so far away that the first correction
+    leaves a residual of about 2^-53 |A| |x0| = 1e-9 of ||b||."""
+    rng = np.random.default_rng(1)
+    return rng.normal(size=nx * ny), 1e6 * rng.normal(size=nx * ny)
+
+
+def _dense(nx, ny):
+    s1 = lambda n: 2.0 * np.eye(n) - np.eye(n, k=1) - np.eye(n, k=-1) - np.diag(np.eye(n)[0] + np.eye(n)[-1])
+    return np.kron(np.eye(ny), s1(nx)) + np.kron(s1(ny), np.eye(nx)) + 0.3 * np.eye(nx * ny)
+
+
+@pytest.mark.parametrize("nx, ny", [(20, 17), (70, 40)])
+def test_iterations_stay_within_maxit(nx, ny, monkeypatch):
+    b, x0 = _far(nx, ny)
+    for passes, maxit, converged in ((None, 1, 0), (None, 2, 1), ("1", 1, 0), ("1", 3, None)):
+        if passes:
+            monkeypatch.setenv("HFH_DIRECT_PASSES", passes)
+        s = _engine(nx, ny)
+        s.set_tolerances(1e-12, 0.0, maxit)
+        _set(s, b, x0)
+        s.solve()
+        assert s.stats()[1] <= maxit
+        assert converged is None or s.stats()[0] == converged
+
+
+# error at most cond(A) rtol of ||x||, as the stopping test allows
+@pytest.mark.parametrize("nx, ny", [(20, 17), (70, 40)])
+def test_krylov_goes_on_where_the_passes_end(nx, ny, monkeypatch):
+    b, x0 = _far(nx, ny)
+    monkeypatch.setenv("HFH_DIRECT_PASSES", "1")
+    s = _engine(nx, ny)
+    _set(s, b, x0)
+    s.solve()
+    assert s.stats()[0] == 1 and s.stats()[1] > 4
+    a = _dense(nx, ny)
+    x = np.linalg.solve(a, b)
+    assert np.linalg.norm(s.get_x() - x) <= np.linalg.cond(a) * 1e-12 * np.linalg.norm(x)
+
+
+def test_member_that_ends_before_another(monkeypatch):
+    # to 1e-13 the 16^2 cavity needs one pass and the 96^2 cavity, in the same
+    # launches, a second one or (with one pass allowed) the Krylov solver
+    runs = []
+    for passes in ("4", "1"):
+        monkeypatch.setenv("HFH_DIRECT_PASSES", passes)
+        b = native.Batch([cases.cavity(n, Re=1.0, dt=1e-3, tempdiscrtype=cases.SEMI_IMPLICIT_EULER, rtol=1e-13,
+                                       atol=0.0, maxit=200) for n in (16, 96)])
+        for _ in range(3):
+            b.step()
+            assert all(b.solve_stats(0, w)["iters"] == 1 and b.solve_stats(0, w)["converged"] for w in range(2))
+        assert b.solve_stats(1)["iters"] in range(2, 5) if passes == "4" else b.solve_stats(1)["iters"] > 4
+        runs.append([b.get(0, f, c) for f, c in ((0, 0), (0, 1), (1, 0), (2, 0))])
+    assert all(np.array_equal(p, q) for p, q in zip(*runs))
+
+
+# the projection and divergence rows are enqueued behind the first pass and run
+# again when that was not the last word; with stage timing on they run once,
+# after the solve
+@pytest.mark.parametrize("make", [
+    lambda **kw: cases.cavity(24, Re=1.0, dt=1e-4, **kw),
+    lambda **kw: cases.cavity(96, Re=1.0, dt=1e-3, tempdiscrtype=cases.SEMI_IMPLICIT_EULER, **kw),
+    lambda **kw: cases.contraction(levels=2, h0=0.25, length=8.0, dt=1e-5, tempdiscrtype=cases.EXPLICIT_EULER, **kw)])
+@pytest.mark.parametrize("passes", ["4", "1"])
+def test_work_enqueued_behind_a_pass_that_was_not_the_last(make, passes, monkeypatch):
+    monkeypatch.setenv("HFH_DIRECT_PASSES", passes)
+    runs = []
+    for timing in (False, True):
+        s = native.Flow(make(rtol=1e-15, atol=0.0, maxit=40))
+        s.set_timing(timing)
+        for _ in range(3):
+            s.step()
+            assert s.solve_stats(0)["iters"] > 1
+        runs.append([s.get(f, c) for f, c in ((0, 0), (0, 1), (1, 0), (2, 0), (3, 0), (3, 1))])
+    assert all(np.array_equal(p, q) for p, q in zip(*runs))
