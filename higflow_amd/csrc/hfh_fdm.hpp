@@ -350,7 +350,9 @@ typedef double fdm_d4 __attribute__((ext_vector_type(4)));
 // round robin) and each holds the whole tile as 2 x 2 matrix-core tiles, so
 // a step of 4 loads feeds 4 MFMAs; the partial tiles meet in LDS.
 // FDM_SCALE divides by the eigenvalue sums (zero for the null mode),
-// FDM_ADD adds the correction to x, with the special unknown's part.
+// FDM_ADD adds the correction to x, with the special unknown's part; a
+// right-hand side that is not finite spreads over the whole system in the
+// products, and x stays what it was.
 template <bool AVEC>
 __global__ void __launch_bounds__(FDM_NT) k_fdm(const int4 *__restrict__ tiles, const FdmJob *__restrict__ jobs,
                                                 const double *__restrict__ mats, const double *__restrict__ lam,
@@ -447,8 +449,11 @@ __global__ void __launch_bounds__(FDM_NT) k_fdm(const int4 *__restrict__ tiles, 
             const bool null = pins[J.sys].pin >= 0 && m == 0 && n == 0;
             dst[o] = null ? 0.0 : v / l;
         } else if (mode == FDM_ADD) {
-            if (pin >= 0) v = (int)o == pin ? zp : v + (mu * g[o] + c);
-            dst[o] += v;
+            if (pin >= 0) {
+                const double t = mu * g[o] + c;
+                v = (int)o == pin && isfinite(t) ? zp : v + t;
+            }
+            if (isfinite(v)) dst[o] += v;
         } else {
             dst[o] = v;
         }
@@ -531,7 +536,7 @@ __global__ void __launch_bounds__(FDM_SNT) k_fdm_small(const FdmSmall *__restric
                                                        int nd, KRows<double> A, const double *__restrict__ mats,
                                                        const double *__restrict__ lam, const double *__restrict__ g,
                                                        const double *__restrict__ dinv, const double *__restrict__ b,
-                                                       double *__restrict__ x, double *__restrict__ bak, double *norms) {
+                                                       double *__restrict__ x, double *norms) {
     extern __shared__ double fdm_lds[];
     __shared__ double sh[3][FDM_SNT / 64];
     __shared__ double s_rp;
@@ -600,9 +605,11 @@ __global__ void __launch_bounds__(FDM_SNT) k_fdm_small(const FdmSmall *__restric
     // the new x stays in LDS (u, without the padding) for its residual
     fdm_small_stage<0>(J, Z[0], w, [&](int m, int n, int, int, double z) {
         const int i = m * nx + n, gi = J.off + i;
-        if (P.pin >= 0) z = i == P.pin ? zp : z + (mu * g[gi] + c);
-        const double x0 = x[gi], xn = x0 + z;
-        bak[gi] = x0;
+        if (P.pin >= 0) {
+            const double t = mu * g[gi] + c;
+            z = i == P.pin && isfinite(t) ? zp : z + t;
+        }
+        const double x0 = x[gi], xn = isfinite(z) ? x0 + z : x0;
         x[gi] = xn;
         u[i] = xn;
     });
@@ -805,12 +812,11 @@ class FdmSolver {
         stages(r, x, psum, dinv, st, true);
     }
 
-    // x += M (b - A x), the x before in bak, and the norms of the new
-    // residual and of b, with one workgroup per system
-    void pass_small(const KRows<double> &A, const double *dinv, const double *b, double *x, double *bak, double *norms,
+    // x += M (b - A x) and the norms of the new residual and of b, with one
+    // workgroup per system
+    void pass_small(const KRows<double> &A, const double *dinv, const double *b, double *x, double *norms,
                     hipStream_t st) {
-        k_fdm_small<<<nsys, FDM_SNT, small_lds_, st>>>(small_.p, pins_.p, nd, A, mats_.p, lam_.p, g_.p, dinv, b, x, bak,
-                                                       norms);
+        k_fdm_small<<<nsys, FDM_SNT, small_lds_, st>>>(small_.p, pins_.p, nd, A, mats_.p, lam_.p, g_.p, dinv, b, x, norms);
     }
 
   private:

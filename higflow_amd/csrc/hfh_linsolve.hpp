@@ -351,7 +351,7 @@ __global__ void __launch_bounds__(BLOCK) k_residual(int n, const int *__restrict
 
 // the same with 4 lanes per row: workgroups of 4 BLOCK threads, one per
 // BLOCK rows, so the partials have k_residual's layout (one per BLOCK rows);
-// prs: the sums of r; xcopy (if given): a copy of x.  LG = 16 takes the rows in four turns of 16 lanes: the
+// prs: the sums of r.  LG = 16 takes the rows in four turns of 16 lanes: the
 // least-squares rows of a 3D mesh (30-65 entries on average, up to 200) wait
 // for their longest row, 49 us on 4 lanes for 47,592 rows, 36 us on 16.
 template <typename T, int LG = 4>
@@ -359,8 +359,7 @@ __global__ void __launch_bounds__(4 * BLOCK) k_residual_l4(int n, const int *__r
                                                            const int *__restrict__ ci, const T *__restrict__ v,
                                                            const T *__restrict__ x, const T *__restrict__ b,
                                                            T *__restrict__ r, T *__restrict__ prr,
-                                                           T *__restrict__ pbb, T *__restrict__ prs,
-                                                           T *__restrict__ xcopy) {
+                                                           T *__restrict__ pbb, T *__restrict__ prs) {
     const int lane = threadIdx.x % LG;
     T rr = 0, bb = 0, rs = 0;
 #pragma unroll
@@ -374,7 +373,6 @@ __global__ void __launch_bounds__(4 * BLOCK) k_residual_l4(int n, const int *__r
         if (i < n && lane == 0) {
             const T bi = b[i], ri = bi - s;
             r[i] = ri;
-            if (xcopy) xcopy[i] = x[i];
             rr += ri * ri;
             bb += bi * bi;
             rs += ri;
@@ -411,8 +409,7 @@ __global__ void __launch_bounds__(4 * BLOCK) k_residual_l4(int n, const int *__r
 template <typename T>
 __global__ void __launch_bounds__(KNT) k_residual_d(int n, KRows<T> A, const T *__restrict__ x,
                                                     const T *__restrict__ b, T *__restrict__ r, T *__restrict__ prr,
-                                                    T *__restrict__ pbb, T *__restrict__ prs, int nb,
-                                                    T *__restrict__ xcopy) {
+                                                    T *__restrict__ pbb, T *__restrict__ prs, int nb) {
     const int i = blockIdx.x * KNT + (int)threadIdx.x;
     const bool in = i < n;
     const int *db = A.dblk + (size_t)blockIdx.x * (KD_MAX + 1);
@@ -441,7 +438,6 @@ __global__ void __launch_bounds__(KNT) k_residual_d(int n, KRows<T> A, const T *
     if (in) {
         const T bi = b[i], ri = bi - s;
         r[i] = ri;
-        if (xcopy) xcopy[i] = x[i];
         rr = ri * ri;
         bb = bi * bi;
         rs = ri;
@@ -906,8 +902,10 @@ class DeviceSystem {
     // its own rounding, where no solver has anything to add.  Every segment is
     // judged by itself: one that has ended keeps its x while the others go
     // on.  False when a segment is left to the Krylov solver (SEG_KRYLOV in
-    // seg_state_), from its best x, after at most `limit` passes; a correction
-    // that is not finite is undone.
+    // seg_state_), from its best x, after at most `limit` passes.  A first
+    // residual that is not finite ends its segment with x as it was, as it
+    // ends a Krylov solve: the corrections leave entries that are not finite
+    // out, so no copy of x is needed before the first pass.
     enum { SEG_OPEN = 0, SEG_FINAL, SEG_KRYLOV };
     bool direct_solve(const double *b, double *x, double rtol, double atol, int limit, int fallback, hipStream_t st,
                       SolveStats &S) {
@@ -919,16 +917,16 @@ class DeviceSystem {
         S.fallback = fallback;
         gs.assign(nseg, S);
         seg_state_.assign(nseg, SEG_OPEN);
-        bool open = true, undone = false, bad = false;
+        bool open = true, undone = false;
         const bool small = fdm.ready && fdm.small;
-        if (!small) true_residual(x, b, st, xbak.p);
+        if (!small) true_residual(x, b, st);
         int pass = 0;
         while (open && pass < limit) {
             pass++;
-            if (pass > 1 && !small)
+            if (pass > 1)
                 HFH_CHECK(hipMemcpyAsync(xbak.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
             if (small) {
-                fdm.pass_small(k64.Av, dinv.p, b, x, xbak.p, norms, st);
+                fdm.pass_small(k64.Av, dinv.p, b, x, norms, st);
             } else {
                 if (fdm.ready)
                     fdm.correct(r.p, x, part3.p, dinv.p, st);
@@ -945,20 +943,17 @@ class DeviceSystem {
             for (int g = 0; g < nseg; g++) {
                 const double rn = std::sqrt(h[2 * g]), bn = std::sqrt(h[2 * g + 1]), tol = std::max(rtol * bn, atol);
                 const double resid = bn > 0 ? rn / bn : rn, old = gs[g].resid;
-                const bool better = seg_state_[g] == SEG_OPEN && std::isfinite(rn) && (pass == 1 || resid < old);
+                const bool better = pass == 1 || (seg_state_[g] == SEG_OPEN && resid < old);
                 back[g] = !better;
                 undo = undo || !better;
                 if (better) {
-                    gs[g].iters = pass;
+                    gs[g].iters = std::isfinite(rn) ? pass : 0;
                     gs[g].resid = resid;
-                    gs[g].converged = rn <= tol;
+                    gs[g].converged = std::isfinite(rn) && rn <= tol;
                 }
                 if (seg_state_[g] != SEG_OPEN) continue;
-                if (gs[g].converged) {
+                if (gs[g].converged || gs[g].iters == 0) {
                     seg_state_[g] = SEG_FINAL;
-                } else if (pass == 1 && !better) {
-                    seg_state_[g] = SEG_KRYLOV;
-                    bad = true;
                 } else if (pass > 1 && !(resid < 0.5 * old)) {
                     stalled.push_back(g);
                 } else {
@@ -981,19 +976,6 @@ class DeviceSystem {
         }
         for (int g = 0; g < nseg; g++)
             if (seg_state_[g] == SEG_OPEN) seg_state_[g] = SEG_KRYLOV;
-        if (bad) {
-            // where the residual was not finite to begin with, x stays what
-            // it was: the Krylov solver would leave it, too
-            true_residual(x, b, st);
-            k_seg_norms<<<nseg, 256, 0, st>>>(segw_.p, part1.p, part2.p, norms);
-            HFH_CHECK(hipStreamSynchronize(st));
-            for (int g = 0; g < nseg; g++) {
-                const double rn = std::sqrt(h[2 * g]), bn = std::sqrt(h[2 * g + 1]);
-                if (gs[g].iters > 0 || std::isfinite(rn)) continue;
-                seg_state_[g] = SEG_FINAL;
-                gs[g].resid = bn > 0 ? rn / bn : rn;
-            }
-        }
         early_done = early && pass == 1 && !undone;
         S.iters = pass;
         return sum_segments(S);
@@ -1060,17 +1042,15 @@ class DeviceSystem {
 
     // r = b - A x and the per-256-row partials of r.r and b.b in part1 /
     // part2: the diagonal-form rows when the FP64 solver has them
-    // (HFH_RESID_DIAG=0: the CSR launch); xcopy (if given) = x
-    void true_residual(const double *x, const double *b, hipStream_t st, double *xcopy = nullptr) {
+    // (HFH_RESID_DIAG=0: the CSR launch)
+    void true_residual(const double *x, const double *b, hipStream_t st) {
         if (k64.Av.dw && resid_diag_)
             k_residual_d<double><<<(n + KNT - 1) / KNT, KNT, 0, st>>>(n, k64.Av, x, b, r.p, part1.p, part2.p,
-                                                                       part3.p, nb, xcopy);
+                                                                       part3.p, nb);
         else if (nnz > 24L * n)
-            k_residual_l4<double, 16><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p,
-                                                                xcopy);
+            k_residual_l4<double, 16><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p);
         else
-            k_residual_l4<double><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p,
-                                                            xcopy);
+            k_residual_l4<double><<<nb, 4 * BLOCK, 0, st>>>(n, rp.p, ci.p, v.p, x, b, r.p, part1.p, part2.p, part3.p);
     }
 
     // FP64 fused solve: Jacobi-PCG (spd) or BiCGStab, warm-started from x.

@@ -516,7 +516,9 @@ __global__ void __launch_bounds__(ND_NT) k_nd_up(const NdTask *__restrict__ task
 }
 
 // Down: x_p = [inv(F11) | -U] [rhs_p ; x_q]; z holds the correction by
-// matrix row for the nodes below, x takes it.
+// matrix row for the nodes below, x takes it.  A right-hand side that is not
+// finite reaches the root of its component and from there every unknown, and
+// x stays what it was.
 __global__ void __launch_bounds__(ND_NT) k_nd_down(const NdTask *__restrict__ tasks, const int *__restrict__ piv,
                                                    const int *__restrict__ border, const double *__restrict__ fac,
                                                    const double *__restrict__ y, double *z, double *__restrict__ x) {
@@ -546,7 +548,7 @@ __global__ void __launch_bounds__(ND_NT) k_nd_down(const NdTask *__restrict__ ta
     nd_dispatch(T, fac, m, nd_v, gather, [&](int row, double s) {
         const int g = piv[T.po + row];
         z[g] = s;
-        x[g] += s;
+        if (isfinite(s)) x[g] += s;
     });
 }
 

@@ -11,14 +11,17 @@ pytestmark = pytest.mark.gpu
 TOL = dict(rtol=1e-11, atol=1e-11, maxit=50000)
 
 
-def _engine(nx, ny):
-    """Five-point Helmholtz rows on nx x ny, solved directly."""
+def _engine(nx, ny, pinned=False):
+    """Five-point rows on nx x ny, solved directly: Helmholtz, or Neumann with
+    the first unknown imposed."""
     s = native.LinearSolver(0, nx * ny)
     s.set_tolerances(1e-12, 0.0, 20000)
     for r in range(nx * ny):
         i, j = r % nx, r // nx
         c = [r + o for o, ok in ((-1, i > 0), (1, i < nx - 1), (-nx, j > 0), (nx, j < ny - 1)) if ok]
-        s.set_Ai(r, c + [r], [-1.0] * len(c) + [len(c) + 0.3])
+        s.set_Ai(r, c + [r], [-1.0] * len(c) + [len(c) + (0.0 if pinned else 0.3)])
+    if pinned:
+        s.impose_value(0, 0.0)
     s.assemble()
     return s
 
@@ -32,14 +35,15 @@ def _set(s, b, x0):
 # one workgroup; tiles
 @pytest.mark.parametrize("nx, ny", [(20, 17), (70, 40)])
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
-def test_right_hand_side_that_is_not_finite(nx, ny, bad):
+@pytest.mark.parametrize("pinned", [False, True])
+def test_right_hand_side_that_is_not_finite(nx, ny, bad, pinned):
     rng = np.random.default_rng(0)
     b, x0 = rng.normal(size=nx * ny), rng.normal(size=nx * ny)
-    fresh = _engine(nx, ny)
+    fresh = _engine(nx, ny, pinned)
     _set(fresh, b, x0)
     fresh.solve()
-    assert fresh.stats()[0] == 1 and fresh.stats()[1] <= 4
-    s = _engine(nx, ny)
+    assert fresh.stats()[1] <= 4
+    s = _engine(nx, ny, pinned)
     worse = b.copy()
     worse[nx * ny // 2] = bad
     _set(s, worse, x0)
@@ -91,6 +95,33 @@ def test_members_beside_one_that_is_not_finite(sides, dim, precision):
         a.step()
         b.step()
         assert not same(range(3))
+
+
+@pytest.mark.parametrize("make", [
+    lambda: cases.contraction(levels=2, h0=0.25, length=8.0, dt=1e-5, tempdiscrtype=cases.EXPLICIT_EULER, **TOL),
+    lambda: cases.wall_layer_cavity(4, levels=1, dt=1e-4, **TOL)])
+def test_refined_mesh_after_a_state_that_is_not_finite(make):
+    case = make()
+    dim = case["dim"]
+    a, b = native.Flow(case), native.Flow(case)
+    for s in (a, b):
+        s.advance(2)
+    state = [(1, 0), (2, 0)] + [(f, d) for f in (0, 3) for d in range(dim)]
+    if case["params"].get("flowtype") == cases.VISCOELASTIC:
+        state += [(6, i * dim + j) for i in range(dim) for j in range(i, dim)]
+    state = [(f, c, a.get(f, c)) for f, c in state]
+    u = state[2][2].copy()
+    u[len(u) // 2] = np.nan
+    b.set(0, 0, u)
+    b.step()
+    # no finite right-hand side: the increment stays the guess
+    assert not b.solve_stats(0)["converged"] and np.isfinite(b.get(2)).all()
+    for s in (a, b):
+        for f, c, v in state:
+            s.set(f, c, v)
+        s.advance(2)
+        assert s.solve_stats(0)["iters"] in range(1, 5)
+    assert all(np.array_equal(a.get(f, c), b.get(f, c)) for f, c, _ in state)
 
 
 def _far(nx, ny):
