@@ -222,7 +222,9 @@ int hfh_slv_assemble_matrix(hfh_slv *s) {
             rp.push_back((int)ci.size());
         }
         const char *ea = std::getenv("HFH_SLV_AMG");  // opt-in V-cycle preconditioning
-        s->sys.set_matrix(rp, ci, v, s->stream, ea && std::strcmp(ea, "1") == 0);
+        const bool amg = ea && std::strcmp(ea, "1") == 0;
+        s->sys.allow_direct = !amg;
+        s->sys.set_matrix(rp, ci, v, s->stream, amg);
         s->db.alloc(s->n);
         s->dx.alloc(s->n);
         s->dirty = false;

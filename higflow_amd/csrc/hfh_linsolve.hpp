@@ -615,6 +615,7 @@ class DeviceSystem {
     double nd_max_flops = 0;
     // the direct solve wants a coupling of at least this share of the diagonal
     double fdm_min_coupling = 0;
+    bool allow_direct = true;
     bool direct() const { return fdm.ready || nd.ready; }
     // work that follows the solve on the stream: a direct solve enqueues it
     // behind its first pass, before the wait; early_done tells whether that
@@ -753,7 +754,7 @@ class DeviceSystem {
             const char *ep = std::getenv("HFH_DIRECT_PASSES");
             direct_passes_ = ep ? std::max(1, std::atoi(ep)) : 4;
             std::vector<int> so = seg_off;
-            const bool on = direct_allowed();
+            const bool on = allow_direct && direct_allowed();
             fdm.ready = on && affordable(fdm, [&] { return fdm.build(hrp, hci, hv, so, st, fdm_min_coupling); });
             // a uniform mesh whose system is left to Jacobi-PCG gets no factors
             nd.ready = on && !fdm.kronecker && nd_max_flops > 0 &&

@@ -199,3 +199,17 @@ def test_work_enqueued_behind_a_pass_that_was_not_the_last(make, passes, monkeyp
             assert s.solve_stats(0)["iters"] > 1
         runs.append([s.get(f, c) for f, c in ((0, 0), (0, 1), (1, 0), (2, 0), (3, 0), (3, 1))])
     assert all(np.array_equal(p, q) for p, q in zip(*runs))
+
+
+def test_engine_that_asks_for_the_v_cycle_gets_it(monkeypatch):
+    b, x0 = _far(70, 40)
+    monkeypatch.setenv("HFH_SLV_AMG", "1")
+    runs = []
+    for direct in (None, "0"):
+        if direct:
+            monkeypatch.setenv("HFH_DIRECT", direct)
+        s = _engine(70, 40)
+        _set(s, b, x0)
+        s.solve()
+        runs.append((s.stats(), s.get_x()))
+    assert runs[0][0] == runs[1][0] and np.array_equal(runs[0][1], runs[1][1])
