@@ -110,6 +110,8 @@ class Flow : public FlowBase {
     }
     ~Flow() override {
         if (host_only_) return;
+        // field writes and the end of a step may still be on their way
+        (void)hipStreamSynchronize(st_);
         for (int s = 0; s < ST_NSTAGE; s++) {
             if (ev0_[s]) (void)hipEventDestroy(ev0_[s]);
             if (ev1_[s]) (void)hipEventDestroy(ev1_[s]);

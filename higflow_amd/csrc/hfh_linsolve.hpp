@@ -560,7 +560,7 @@ struct HostStage {
                 at = 0;
             }
             std::memcpy(p + at, src, b);
-            k_copy<double><<<nblocks((long)k), BLOCK, 0, st>>>((int)k, reinterpret_cast<double *>(p + at), dst);
+            copy(reinterpret_cast<double *>(p + at), dst, k, st);
             at += (b + 63) / 64 * 64;
             dst += k;
             src += k;
@@ -572,14 +572,24 @@ struct HostStage {
         open();
         while (n > 0) {
             const size_t k = std::min(n, CAP / sizeof(double)), b = k * sizeof(double);
-            k_copy<double><<<nblocks((long)k), BLOCK, 0, st>>>((int)k, src, reinterpret_cast<double *>(p));
+            copy(src, reinterpret_cast<double *>(p), k, st);
             HFH_CHECK(hipStreamSynchronize(st));
+            at = 0;
             std::memcpy(dst, p, b);
             dst += k;
             src += k;
             n -= k;
         }
-        at = 0;
+    }
+
+  private:
+    // a copy that could not be launched is an error here: the buffer would
+    // still hold what an earlier exchange left
+    static void copy(const double *src, double *dst, size_t k, hipStream_t st) {
+        int n = (int)k;
+        void *args[] = {&n, &src, &dst};
+        HFH_CHECK(hipLaunchKernel(reinterpret_cast<const void *>(k_copy<double>), dim3(nblocks(n)), dim3(BLOCK), args, 0,
+                                  st));
     }
 };
 
