@@ -358,6 +358,8 @@ class Flow : public FlowBase {
         DevBuf<float> sval32;
         std::vector<int4> htask;
         int ntask = 0, gen0 = 0, sell0 = 0, out0 = -1;
+        long task_bytes = 0;  // tasks, templates and other rows as a launch streams them
+        long const_rows = 0;  // rows whose constants it reads
         bool has_y = false, f32 = false;
         std::vector<int> order;  // device row k is the group's row order[k]
     } dDu_, dK_, dCv_, dMom_, dDiv_, dGrad_;
@@ -490,6 +492,9 @@ class Flow : public FlowBase {
     // one launch of a group: the operator as uploaded, then per (row,
     // component) the constant, the destination index and the write
     static long gdbytes(const DGroup &dg) {
+        if (dg.ntask > 0)
+            return dg.task_bytes + dg.const_rows * (dg.f32 ? 4 : 8) + (dg.out0 < 0 ? 4L * dg.nrow : 0) +
+                   8L * dg.nrow * dg.ncomp;
         return dg.nrow ? dg.op_bytes + (long)dg.nrow * dg.ncomp * (8 + 4 + 8) : 0;
     }
     void refold_constants();

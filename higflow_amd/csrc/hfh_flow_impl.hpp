@@ -234,11 +234,6 @@ void Flow<D>::upload_device() {
         dGrad_.y.upload(y.data(), y.size(), st_);
         HFH_CHECK(hipStreamSynchronize(st_));  // y is a local
     }
-    // algorithmic bytes of the interpolation stages with the operators as
-    // uploaded (template rows or CSR)
-    bytes_[ST_INTERP] = gdbytes(dMom_) + gdbytes(dDu_) + gdbytes(dK_) + gdbytes(dCv_);
-    bytes_[ST_DIV] = gdbytes(dDiv_);
-    bytes_[ST_PROJECT] = gdbytes(dGrad_) + (long)dGrad_.nrow * 12 + (long)Nc_ * 24;
     {
         const char *ex = std::getenv("HFH_EXTRAP");
         extrap_ = ex ? std::max(0, std::min(2, std::atoi(ex))) : 2;
@@ -318,6 +313,11 @@ void Flow<D>::upload_device() {
         }
     }
     refold_constants();
+    // algorithmic bytes of the interpolation stages with the operators as
+    // uploaded (wave tasks, template rows or CSR)
+    bytes_[ST_INTERP] = gdbytes(dMom_) + gdbytes(dDu_) + gdbytes(dK_) + gdbytes(dCv_);
+    bytes_[ST_DIV] = gdbytes(dDiv_);
+    bytes_[ST_PROJECT] = gdbytes(dGrad_) + (long)dGrad_.nrow * 12 + (long)Nc_ * 24;
     HFH_CHECK(hipStreamSynchronize(st_));
 }
 
@@ -499,6 +499,9 @@ void Flow<D>::upload_group(DGroup &dg, const Group &g, int, int out_stride, bool
         k = e;
     }
     dg.gen0 = gen0;
+    const long ws = f32 ? 4 : 8;  // bytes of a weight
+    long tb = (long)dg.ntempl * (4 + GT_MAX * (4 + ws));
+    for (const int4 &t : task) tb += t.w < 0 ? 4L * t.z : 0;
     // the other rows, the longest first: the least-squares rows of a 3D mesh
     // (about 100 entries, sums of them more) on 16 lanes when they are the
     // bulk, the rest column by column
@@ -512,6 +515,8 @@ void Flow<D>::upload_group(DGroup &dg, const Group &g, int, int out_stride, bool
     if (padded > INT_MAX) return;
     dg.sell0 = sell0;
     const int ng = dg.nrow - sell0;
+    for (int k = gen0; k < sell0; k++) tb += 8 + (pcode[k] >= 0 ? 0 : 8 + length(k) * (4 + ws));
+    tb += padded * (4 + ws) + 4L * ng;
     if (ng > 0) {
         std::vector<int> slen(ng), scol(padded, 0);
         std::vector<double> sval(padded, 0.0);
@@ -544,6 +549,7 @@ void Flow<D>::upload_group(DGroup &dg, const Group &g, int, int out_stride, bool
     }
     if (task.empty()) return;
     dg.ntask = (int)task.size();
+    dg.task_bytes = tb + dg.ntask * (long)(sizeof(int4) + sizeof(int));
     dg.task.upload(task.data(), task.size(), st_);
     dg.czero.alloc(task.size());
     dg.htask.swap(task);
@@ -678,12 +684,14 @@ void Flow<D>::refold_constants() {
         }
         const std::vector<double> &c = keep.back();
         if (p.d->ntask > 0) {
+            p.d->const_rows = p.d->sell0 - p.d->gen0;
             keepz.emplace_back(p.d->ntask);
             for (int w = 0; w < p.d->ntask; w++) {
                 const int4 &t = p.d->htask[w];
                 bool zero = true;
                 for (int r = t.y; r < t.y + t.z && zero; r++) zero = c[r] == 0.0;
                 keepz.back()[w] = zero;
+                if (!zero) p.d->const_rows += t.z;
             }
             p.d->czero.upload(keepz.back().data(), keepz.back().size(), st_);
         }
