@@ -57,6 +57,25 @@ def test_pressure_of_a_refined_mesh(which, monkeypatch):
     assert np.linalg.norm(x - y) <= _cond(a, 0) * (sa["resid"] + sb["resid"]) * np.linalg.norm(y)
 
 
+# the same in the residuals, where no condition number enters (on the 3D meshes
+# it makes the bound above loose): ||A (x - y)|| <= (ra + rb) ||b|| and, for
+# either residual as computed, its rounding (len + 2) u || |A||x| + |b| ||, with
+# ||b|| <= ||A y|| / (1 - rb) and |b| <= |A||x| but for ra
+@pytest.mark.parametrize("make", [lambda **kw: cases.wall_layer_cavity(4, levels=1, dt=1e-4, **kw),
+                                  lambda **kw: cases.wall_layer_cavity(6, levels=2, dt=1e-4, **kw),
+                                  lambda **kw: cases.contraction(levels=2, h0=0.25, length=8.0, dt=1e-5,
+                                                                 tempdiscrtype=cases.EXPLICIT_EULER, **kw)])
+def test_residual_of_the_difference(make, monkeypatch):
+    a, b = _pair(make(rtol=RTOL, atol=0.0, maxit=50000), monkeypatch)
+    rp, ci, v, _ = a.operator(0)
+    m = sp.csr_matrix((v, ci, rp))
+    x, y = a.get(2), b.get(2)
+    ra, rb = a.solve_stats(0)["resid"], b.solve_stats(0)["resid"]
+    bn = np.linalg.norm(m @ y) / (1.0 - rb)
+    rounding = np.linalg.norm((np.diff(rp) + 3) * 2.0 ** -53 * (abs(m) @ np.maximum(abs(x), abs(y))))
+    assert np.linalg.norm(m @ (x - y)) <= (ra + rb) * bn + 2 * rounding
+
+
 def test_velocity_blocks_of_a_large_mixed_run(monkeypatch):
     case = cases.contraction(levels=4, graded=True, h0=0.05, dt=1e-5, rtol=RTOL, atol=0.0, maxit=50000)
     a, b = _pair(case, monkeypatch, precision=1, inner_rtol=1e-5)
