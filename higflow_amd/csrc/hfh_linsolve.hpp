@@ -775,6 +775,8 @@ class DeviceSystem {
                                  fdm.ready ? "fast diagonalisation" : nd.ready ? "nested dissection" : "Krylov",
                                  nd.flops, nd.entries);
         }
+        if (direct() && (int)segback_.n < nseg) segback_.alloc(nseg);
+        if (direct() && nseg > 1 && (int)xkeep_.n < n) xkeep_.alloc(n);
         k64.defer_amg = k32.defer_amg = direct() && k64.want_amg;
         hrp_.clear();
         hci_.clear();
@@ -996,7 +998,6 @@ class DeviceSystem {
     // device first: read from there by each workgroup, host memory costs more
     // than the copies.
     void put_back(const double *from, double *x, hipStream_t st) {
-        if ((int)segback_.n < nseg) segback_.alloc(nseg);
         HFH_CHECK(hipMemcpyAsync(segback_.p, hpin_ + off_bk_, nseg * sizeof(int), hipMemcpyHostToDevice, st));
         k_seg_copy<<<nb, BLOCK, 0, st>>>(n, rp.p, nseg > 1 ? bseg_.p : nullptr, segback_.p, from, x);
     }
@@ -1030,7 +1031,6 @@ class DeviceSystem {
         bool keep = false;
         for (int q : state) keep = keep || q == SEG_FINAL;
         if (keep) {
-            if ((int)xkeep_.n < n) xkeep_.alloc(n);
             HFH_CHECK(hipMemcpyAsync(xkeep_.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, st));
         }
         SolveStats K = krylov(maxit - S.iters);
