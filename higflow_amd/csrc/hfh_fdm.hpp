@@ -23,10 +23,10 @@
 // correction leaves rounding, so it is normally the only one.
 //
 // Measured on MI355X, 20 steps between two field exchanges, Krylov with the
-// V-cycle against this: cavity 64^2 12.6 -> 1.9 ms, cavity 256^2
-// 29.1 -> 3.3 ms, Oldroyd-B cavity 512^2 63.6 -> 16.5 ms, 64-cavity sweep
-// 194 -> 53 ms, 3D 15^3 22.7 -> 6.4 ms; one 256^2 Poisson solve of the
-// engine (Jacobi-BiCGStab, 1521 iterations) 26.4 -> 0.18 ms.
+// V-cycle against this: cavity 64^2 12.8 -> 1.7 ms, cavity 256^2
+// 29.4 -> 2.6 ms, Oldroyd-B cavity 512^2 63 -> 11.4 ms, 64-cavity sweep
+// 190 -> 40.5 ms, 3D 15^3 (pressure only) 22.1 -> 8.1 ms; one 256^2 Poisson
+// solve of the engine (Jacobi-BiCGStab, 1521 iterations) 27.5 -> 0.17 ms.
 #pragma once
 #include <hip/hip_runtime.h>
 

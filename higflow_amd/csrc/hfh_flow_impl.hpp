@@ -247,20 +247,31 @@ void Flow<D>::upload_device() {
         if (!momRe_[d].empty()) dMomRe_[d].upload(momRe_[d].data(), momRe_[d].size(), st_);
     if (!vePar_.empty()) dVePar_.upload(vePar_.data(), vePar_.size(), st_);
     // Factors of refined meshes (hfh_nd.hpp): for explicit runs, and for
-    // large semi-implicit runs in the mixed form, where they replace FP32
-    // refinements that end well below the tolerance.  FP64 iterations stop at
-    // the tolerance; the error they leave in u*, over dt, is 1e-9 of the
-    // pressure (3-level contraction, tolerance 1e-11, against runs at 1e-13),
-    // and semi-implicit runs whose systems are solved by them (all of the
-    // FP64 form, small ones of the mixed form) keep them and their results.
+    // semi-implicit runs in the mixed form from 65,536 cells up.  This line
+    // keeps results, it is not where the speed or the accuracy changes sides:
+    // a run's fields stay within 1e-9 of those of the iterations it was set
+    // up for.  These stop at the tolerance, and the error they leave in u*,
+    // over dt, is 1e-10 to 2.6e-9 of the pressure, 1e-13 with the factors.
+    // Contractions, 25 steps to 1e-11 against runs to 1e-13, error of p and
+    // ms per step of the iterations and of the factors: FP64, 19,936 cells
+    // 3.5e-10, 2.99 and 7e-14, 0.46; 47,800 cells 3.5e-10, 5.54 and 3e-14,
+    // 0.66; 77,440 cells 2.4e-10, 10.5 and 5e-14, 0.71; mixed form 3.0e-10,
+    // 3.12; 1.4e-10, 5.20; 1.0e-10, 8.56 (the factors as in FP64).  From
+    // loaded states p of the 47,800-cell FP64 run moved by up to 2.6e-9, of
+    // the 121,000-cell mixed run (18.5 ms per 20 steps against 229) by 1e-10;
+    // the line lies between these two.  Set-up takes 0.2 to 0.5 s longer at
+    // 12,048 to 121,000 cells (the hierarchy is not built): 70 steps of the
+    // 12^3 wall layer.
     const bool semi = par_.tempdiscrtype == SEMI_IMPLICIT_EULER;
     const bool factors = !semi || (par_.precision == 1 && Nc_ >= 65536);
     psys_.nd_max_flops = hsysB_.nd_max_flops = factors ? 2e11 : 0;
     // the same for nearly diagonal velocity systems of uniform meshes (no
     // coupling at the strength threshold, so no hierarchy either), which
-    // converge in 2-7 Jacobi-PCG iterations: at a coupling of 0.05 and
-    // Re = 160 the direct solve moved the pressure by 2e-9, at 0.09 and above
-    // by 2.4e-10 at most
+    // converge in 4 to 10 Jacobi-PCG iterations: the direct solve would move
+    // fields by up to 1e-9 towards the runs to 1e-13 (couplings 0.01 to 0.07:
+    // 64^2 and 256^2 p 6e-11 to 5e-10, 3D 15^3 u 2e-10 to 1e-9; with it all
+    // within 1e-13) and take 0.14 ms per step instead of 0.20-0.27 (64^2),
+    // 0.18 instead of 0.23-0.29 (256^2), 0.23 instead of 0.32-0.41 (15^3)
     hsysB_.fdm_min_coupling = 0.08;
     psys_.set_matrix(Arp_, Aci_, Av_, st_, true, pseg_);
     if (par_.tempdiscrtype == SEMI_IMPLICIT_EULER) {

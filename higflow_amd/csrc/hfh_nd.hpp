@@ -13,9 +13,10 @@
 // with W = F21 inv(F11), U = inv(F11) F12 of each front.
 //
 // Measured on MI355X (20 steps; 10 in 3D), against AMG-BiCGStab and FP32
-// refinement: graded 4-level contraction, mixed form, 226 -> 19 ms;
-// 12^3 wall-layer cavity 56 -> 7.3 ms, where a solve reads 0.57 GB of factors
-// (host factors: 1.5e11 operations, 4 s on 8 cores).
+// refinement: graded 4-level contraction, mixed form, 229 -> 18.5 ms;
+// 12^3 wall-layer cavity 56 -> 7.0 ms, where a solve reads 0.57 GB of factors
+// (host factors: 1.5e11 operations, 4 s on 8 cores; on 16, the set-up takes
+// 5.3 s with them and 5.1 with the V-cycle hierarchy in their place).
 #pragma once
 #include <hip/hip_runtime.h>
 
