@@ -453,7 +453,8 @@ __global__ void __launch_bounds__(FDM_NT) k_fdm(const int4 *__restrict__ tiles, 
                 const double t = mu * g[o] + c;
                 v = (int)o == pin && isfinite(t) ? zp : v + t;
             }
-            if (isfinite(v)) dst[o] += v;
+            const double x0 = dst[o];
+            dst[o] = isfinite(v) ? x0 + v : x0;
         } else {
             dst[o] = v;
         }

@@ -548,8 +548,9 @@ __global__ void __launch_bounds__(ND_NT) k_nd_down(const NdTask *__restrict__ ta
     };
     nd_dispatch(T, fac, m, nd_v, gather, [&](int row, double s) {
         const int g = piv[T.po + row];
+        const double x0 = x[g];
         z[g] = s;
-        if (isfinite(s)) x[g] += s;
+        x[g] = isfinite(s) ? x0 + s : x0;
     });
 }
 
