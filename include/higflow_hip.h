@@ -201,7 +201,8 @@ int hfh_last_solve(hfh_solver *s, int *iters, double *resid, int *outer);
  * converged (higtree/src/solver.h:80-82): info = {iterations, refinement
  * steps, mixed form's FP64 use (0 FP32 refinement, 1 FP32 failed and the
  * solve finished in FP64, 2 FP64 chosen as the faster form), true-residual
- * restarts}; a direct solve reports its passes (1 to 4) as iterations;
+ * restarts}; a direct solve reports its passes as iterations (1 to 4, 0 when
+ * the right-hand side is not finite, more when the Krylov solver went on);
  * returns 1 converged, 0 not converged, <0 error */
 int hfh_solve_stats(hfh_solver *s, int which, int *info, double *resid);
 
